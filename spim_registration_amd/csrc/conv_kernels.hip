@@ -1,4 +1,7 @@
-// FFT convolution passes of one block (window) of a volume, for gfx950.
+// FFT convolution passes of one block (window) of a volume, for gfx950: the
+// choice of the kernels by length, and the LDS kernels for the lengths that
+// neither the fixed-length register kernels (fft_fast.hip) nor the two-radix
+// ones (fft_any.h) take.
 //
 // A 3D real convolution with circular wrap over the padded size q is done in
 // four launches over a half spectrum S laid out [z][y][kx], kx in [0, q.x/2]:
@@ -154,6 +157,8 @@ struct ZParams {
   const float2* kspec;
   float2* aux;  // with kspec: the forward spectrum before the product, all rows (nullable)
   const float2* pre;  // with kspec: the lines' spectrum already transformed along z (nullable)
+  const double* wsum;  // with pre: the product's zero-frequency value is *wsum kdc (nullable)
+  double kdc;
   float scale, dir;
   int hx, pitch, qy, qz, zlo, zhi, lines;
   FftPlan plan;
@@ -184,7 +189,9 @@ __device__ __forceinline__ void z_body(const ZParams& P, int bx, int by) {
       if (c0 + b < P.hx) {
         const float2 v = buf[z * lp + b];
         if (P.aux) gmem(P.aux)[z * plane + col + b] = v;
-        buf[z * lp + b] = cmul(v, gmem(P.kspec)[z * plane + col + b]);
+        float2 y = cmul(v, gmem(P.kspec)[z * plane + col + b]);
+        if (P.wsum && by == 0 && c0 + b == 0 && z == 0) y = make_float2((float)(*gmem(P.wsum) * P.kdc), 0.f);
+        buf[z * lp + b] = y;
       }
     }
     __syncthreads();
@@ -437,6 +444,7 @@ __global__ __launch_bounds__(kThreads) void k_x_inverse_batch(const XInvParams* 
 hipError_t launch_x_forward(const ShapePlan& sp, const ConvGeom& g, const float* src, int gather, float2* spec,
                             hipStream_t stream) {
   if (fast_size(g.q.x / 2)) return launch_x_forward_fast(sp, g, src, gather, spec, stream);
+  if (any_size(sp.px)) return launch_x_forward_any(sp, g, src, gather, spec, stream);
   XFwdParams P;
   P.g = g;
   P.src = src;
@@ -459,7 +467,8 @@ hipError_t launch_x_forward(const ShapePlan& sp, const ConvGeom& g, const float*
 hipError_t launch_y(const ShapePlan& sp, float2* spec, int zlo, int zhi, int ylo, int yhi, float dir,
                     hipStream_t stream) {
   if (zhi <= zlo) return hipSuccess;
-  if (fast_size(sp.q.y)) return launch_y_fast(sp, spec, zlo, zhi, ylo, yhi, dir, stream);
+  if (register_size(sp.py))
+    return launch_y_window(sp, spec, zlo, zhi, ylo, yhi, dir, {0, 0, 0}, {1 << 30, 1 << 30, 1 << 30}, stream);
   YParams P;
   P.spec = spec;
   P.hx = sp.hx;
@@ -479,12 +488,23 @@ hipError_t launch_y(const ShapePlan& sp, float2* spec, int zlo, int zhi, int ylo
   return hipGetLastError();
 }
 
+hipError_t launch_y_window(const ShapePlan& sp, float2* spec, int zlo, int zhi, int ylo, int yhi, float dir,
+                           Int3 in_lo, Int3 in_hi, hipStream_t stream) {
+  if (zhi <= zlo) return hipSuccess;
+  if (fast_size(sp.q.y)) return launch_y_fast_window(sp, spec, zlo, zhi, ylo, yhi, dir, in_lo, in_hi, stream);
+  if (any_size(sp.py)) return launch_y_any(sp, spec, zlo, zhi, ylo, yhi, dir, in_lo, in_hi, stream);
+  return hipErrorInvalidValue;
+}
+
 hipError_t launch_z(const ShapePlan& sp, float2* spec, const float2* kspec, float scale, int zlo, int zhi,
-                    hipStream_t stream, float dir, float2* aux, const float2* pre) {
-  if (fast_size(sp.q.z)) return launch_z_fast(sp, spec, kspec, scale, zlo, zhi, stream, dir, aux, pre);
+                    hipStream_t stream, float dir, float2* aux, const float2* pre, const double* wsum, double kdc) {
+  if (fast_size(sp.q.z)) return launch_z_fast(sp, spec, kspec, scale, zlo, zhi, stream, dir, aux, pre, wsum, kdc);
+  if (any_size(sp.pz)) return launch_z_any(sp, spec, kspec, scale, zlo, zhi, stream, dir, aux, pre, wsum, kdc);
   ZParams P;
   P.aux = aux;
   P.pre = pre;
+  P.wsum = pre ? wsum : nullptr;
+  P.kdc = kdc;
   P.dir = dir;
   P.spec = spec;
   P.kspec = kspec;
@@ -506,8 +526,8 @@ hipError_t launch_z(const ShapePlan& sp, float2* spec, const float2* kspec, floa
 }
 
 bool z_grad_supported(const ShapePlan& sp) {
-  // generic lengths: two line sets of sp.bz lines in LDS
-  return fast_size(sp.q.z) || sizeof(float2) * (sp.q.z + 2 * (size_t)sp.q.z * (sp.bz + 1)) <= 64 * 1024;
+  // LDS kernels: two line sets of sp.bz lines
+  return register_size(sp.pz) || sizeof(float2) * (sp.q.z + 2 * (size_t)sp.q.z * (sp.bz + 1)) <= 64 * 1024;
 }
 
 hipError_t launch_z_grad(const ShapePlan& sp, float2* spec, const float2* what, const float2* khat, float2* corr,
@@ -516,6 +536,8 @@ hipError_t launch_z_grad(const ShapePlan& sp, float2* spec, const float2* what, 
   if (!z_grad_supported(sp) || zlo < 0 || zhi > sp.q.z || kz < 0 || kz > sp.q.z) return hipErrorInvalidValue;
   if (fast_size(sp.q.z))
     return launch_z_fast_grad(sp, spec, what, khat, corr, mode, first, shift, zlo, zhi, kz, rsum, adj, adj_add, stream);
+  if (any_size(sp.pz))
+    return launch_z_any_grad(sp, spec, what, khat, corr, mode, first, shift, zlo, zhi, kz, rsum, adj, adj_add, stream);
   ZGradParams P{};
   P.rsum = rsum;
   P.adj = adj;
@@ -547,7 +569,9 @@ hipError_t launch_z_grad(const ShapePlan& sp, float2* spec, const float2* what, 
 
 int x_inverse_workgroups(const ShapePlan& sp, const ConvGeom& g) {
   const int nrows = g.eff_size.y * g.eff_size.z;
-  const int rows = fast_size(g.q.x / 2) ? x_fast_rows_per_wg(g.q.x / 2) : sp.bx;
+  const int rows = fast_size(g.q.x / 2) ? x_fast_rows_per_wg(g.q.x / 2)
+                   : any_size(sp.px)    ? x_any_rows_per_wg(sp.px)
+                                        : sp.bx;
   return (nrows + rows - 1) / rows;
 }
 
@@ -567,6 +591,7 @@ hipError_t launch_x_inverse(const ShapePlan& sp, const ConvGeom& g, const float2
   if (nwg) *nwg = n;
   if (n == 0) return hipSuccess;
   if (fast_size(M)) return launch_x_inverse_fast(sp, g, spec, e, stream, n);
+  if (any_size(sp.px)) return launch_x_inverse_any(sp, g, spec, e, stream, n);
   size_t lds = sizeof(float2) * (g.q.x + (size_t)(M + 1) * (P.lines + 1));
   (void)hipGetLastError();  // launch errors only, not a stale one
   hipLaunchKernelGGL(k_x_inverse, dim3(n), dim3(kThreads), lds, stream, P);
@@ -599,7 +624,33 @@ hipError_t launch_yx_inverse_passes(const ShapePlan& sp, const ConvGeom& g, floa
 }
 
 // ---------------------------------------------------------------------------
-// batched generic passes
+// batched passes of the register kernels of any length
+
+bool pass_is_any(const PassDesc& d) {
+  switch (d.kind) {
+    case kPassXForward:
+    case kPassXInverse: return any_size(d.sp->px);
+    case kPassYForward:
+    case kPassYInverse: return any_size(d.sp->py);
+    case kPassZConv: return any_size(d.sp->pz) && d.kspec;
+  }
+  return false;
+}
+
+int build_any_params(const PassDesc& d, void* out, int* gx, int* gy, int* cls, int* threads, size_t* lds) {
+  if (d.kind == kPassXForward || d.kind == kPassXInverse) return build_any_x_params(d, out, gx, gy, cls, threads, lds);
+  return build_any_yz_params(d, out, gx, gy, cls, threads, lds);
+}
+
+hipError_t launch_batch_any(int kind, int cls, int epi, const void* items, const int* prefix, const int* gx, int nitems,
+                            int nwg, int threads, size_t lds, hipStream_t stream) {
+  if (kind == kPassXForward || kind == kPassXInverse)
+    return launch_batch_any_x(kind, cls, epi, items, prefix, gx, nitems, nwg, threads, lds, stream);
+  return launch_batch_any_yz(kind, cls, items, prefix, gx, nitems, nwg, threads, lds, stream);
+}
+
+// ---------------------------------------------------------------------------
+// batched LDS passes
 
 int build_generic_params(const PassDesc& d, void* out, int* gx, int* gy, size_t* lds) {
   const ShapePlan& sp = *d.sp;
@@ -646,6 +697,7 @@ int build_generic_params(const PassDesc& d, void* out, int* gx, int* gy, size_t*
       ZParams P{};
       P.aux = nullptr;
       P.pre = nullptr;
+      P.wsum = nullptr;
       P.spec = d.spec;
       P.kspec = d.kspec;
       P.scale = d.scale;

@@ -23,6 +23,7 @@ struct FftPlan {
   int radix[kMaxPasses];
   int ns[kMaxPasses];    // product of the radices of the earlier passes
   unsigned magic[kMaxPasses];  // ceil(2^32 / ns) for ns > 1: j / ns = umulhi(j, magic) for j * ns < 2^32
+  int a = 0, b = 0;      // n = a b for the two-pass register kernels (fft_any.h), 0: no such split
 };
 
 __device__ __forceinline__ float2 cmul(float2 a, float2 b) {

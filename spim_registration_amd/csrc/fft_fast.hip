@@ -159,6 +159,9 @@ struct ZFastParams {
   // with kspec (single launches only): the lines' spectrum already
   // transformed along z, in place of spec (nullable)
   const float2* pre = nullptr;
+  // with pre: the product's zero-frequency value is *wsum kdc (nullable)
+  const double* wsum = nullptr;
+  double kdc = 0.0;
 };
 
 template <int N>
@@ -222,6 +225,7 @@ __device__ __forceinline__ void z_fast_body(const ZFastParams& P, int bx, int by
     }
 #pragma unroll
     for (int i = 0; i < E; ++i) v[i] = cmul(v[i], kv[i]);
+    if (P.wsum && by == 0 && col == 0 && jt == 0) v[0] = make_float2((float)(*gmem(P.wsum) * P.kdc), 0.f);
     fft_reverse_order<N>(v, lds, jt, tw, 1, 1.f, addr);
     if (valid) {
 #pragma unroll
@@ -1234,8 +1238,10 @@ hipError_t launch_y_fast(const ShapePlan& sp, float2* spec, int zlo, int zhi, in
 }
 
 hipError_t launch_z_fast(const ShapePlan& sp, float2* spec, const float2* kspec, float scale, int zlo, int zhi,
-                         hipStream_t stream, float dir, float2* aux, const float2* pre) {
-  ZFastParams P{spec, kspec, sp.tw_z, scale, dir, sp.hx, sp.pitch, sp.q.y, zlo, zhi, nullptr, nullptr, 0, aux, pre};
+                         hipStream_t stream, float dir, float2* aux, const float2* pre, const double* wsum,
+                         double kdc) {
+  ZFastParams P{spec, kspec, sp.tw_z, scale, dir, sp.hx, sp.pitch, sp.q.y, zlo, zhi, nullptr, nullptr, 0, aux, pre,
+                pre ? wsum : nullptr, kdc};
   (void)hipGetLastError();
 #define MVD_Z(N)                                                                                \
   case N: {                                                                                     \

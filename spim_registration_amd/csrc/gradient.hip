@@ -237,6 +237,52 @@ hipError_t launch_set_dc(float2* spec, const double* v, hipStream_t stream) {
   return hipGetLastError();
 }
 
+// How many positions q of [lo, lo + wd) have p as their mirror-single image
+// (period 2n - 2: q = p or -p modulo the period).
+__device__ __forceinline__ int window_count(int p, int lo, int wd, int n) {
+  if (n == 1) return wd;
+  const int period = 2 * n - 2;
+  // integers = r mod period in [lo, lo + wd)
+  auto count = [&](int r) {
+    const int first = ((r - lo) % period + period) % period;  // from lo to the first of them
+    return first < wd ? (wd - 1 - first) / period + 1 : 0;
+  };
+  return count(p) + (p == 0 || p == n - 1 ? 0 : count(-p));
+}
+
+// Partials (double) of the sum of a window of the mirror-extended image: the
+// exact zero-frequency value of the window's spectrum.  A workgroup takes
+// image rows; a thread keeps the counts of its columns.
+__global__ __launch_bounds__(kGThreads) void k_window_sum(const float* img, Int3 n, Int3 lo, Int3 wd, double* part) {
+  __shared__ double rs[kGThreads];
+  double s = 0.0;
+  for (int x = threadIdx.x; x < n.x; x += kGThreads) {
+    double col = 0.0;
+    for (int row = blockIdx.x; row < n.y * n.z; row += gridDim.x) {
+      const int z = row / n.y, y = row - z * n.y;
+      const int c = window_count(y, lo.y, wd.y, n.y) * window_count(z, lo.z, wd.z, n.z);  // uniform
+      col += (double)c * (double)img[(int64_t)row * n.x + x];
+    }
+    s += col * (double)window_count(x, lo.x, wd.x, n.x);
+  }
+  rs[threadIdx.x] = s;
+  __syncthreads();
+  for (int o = kGThreads / 2; o > 0; o >>= 1) {
+    if (threadIdx.x < o) rs[threadIdx.x] += rs[threadIdx.x + o];
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) part[blockIdx.x] = rs[0];
+}
+
+hipError_t launch_window_sum_to(const float* img, Int3 n, Int3 lo, Int3 wd, double* part, int nparts, double* out,
+                                hipStream_t stream) {
+  (void)hipGetLastError();
+  hipLaunchKernelGGL(k_window_sum, dim3(nparts), dim3(kGThreads), 0, stream, img, n, lo, wd, part);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  return launch_reduce_sum(part, nparts, out, stream);
+}
+
 // The same fold as a gather over the image voxels the window covers (its
 // direct box [a, b)): per voxel, the window positions whose mirror-single
 // image it is -- the direct one and, near a face the window crosses, the one

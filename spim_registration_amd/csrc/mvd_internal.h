@@ -238,9 +238,16 @@ hipError_t launch_y(const ShapePlan& sp, float2* spec, int zlo, int zhi, int ylo
 // (kernel spectra, gradient passes).  aux (with kspec): also store the forward
 // spectrum before the product, all rows.  pre (with kspec): the lines are
 // read from pre, already transformed along z (no forward transform); the
-// output rows still go to spec.
+// output rows still go to spec.  wsum (with pre; nullable): the zero-frequency
+// value of the product is *wsum kdc, computed in double.
 hipError_t launch_z(const ShapePlan& sp, float2* spec, const float2* kspec, float scale, int zlo, int zhi,
-                    hipStream_t stream, float dir = -1.f, float2* aux = nullptr, const float2* pre = nullptr);
+                    hipStream_t stream, float dir = -1.f, float2* aux = nullptr, const float2* pre = nullptr,
+                    const double* wsum = nullptr, double kdc = 0.0);
+// y pass whose input holds data only in rows [in_lo.y, in_hi.y) of planes
+// [in_lo.z, in_hi.z); every other input row is read as zero (register_size
+// lengths).
+hipError_t launch_y_window(const ShapePlan& sp, float2* spec, int zlo, int zhi, int ylo, int yhi, float dir,
+                           Int3 in_lo, Int3 in_hi, hipStream_t stream);
 // Gradient z pass (z_grad_supported): forward R^ of the
 // y-transformed residual in spec; adjoint R^ conj(P^) inverted into rows
 // [zlo, zhi) of spec; correlation conj(R^) W^ with the lag shift `shift`
@@ -297,17 +304,32 @@ hipError_t launch_weight_normalize(float* weights, int nviews, int64_t n, int64_
                                    hipStream_t stream);
 hipError_t launch_osem_scale(float* weights, int64_t n, float osem, hipStream_t stream);
 
-// Register-resident kernels for power-of-two lengths (fft_fast.hip).
+// Two-pass register kernels for any length with a split into two radices
+// (fft_any_x.hip, fft_any_yz.hip).
+inline bool any_size(const FftPlan& p) { return p.a > 0; }
+int x_any_rows_per_wg(const FftPlan& p);
+hipError_t launch_y_any(const ShapePlan& sp, float2* spec, int zlo, int zhi, int ylo, int yhi, float dir, Int3 in_lo,
+                        Int3 in_hi, hipStream_t stream);
+hipError_t launch_z_any(const ShapePlan& sp, float2* spec, const float2* kspec, float scale, int zlo, int zhi,
+                        hipStream_t stream, float dir, float2* aux, const float2* pre, const double* wsum, double kdc);
+hipError_t launch_z_any_grad(const ShapePlan& sp, float2* spec, const float2* what, const float2* khat, float2* corr,
+                             int mode, int first, Int3 shift, int zlo, int zhi, int kz, const double* rsum,
+                             float2* adj, bool adj_add, hipStream_t stream);
+hipError_t launch_x_forward_any(const ShapePlan& sp, const ConvGeom& g, const float* src, int gather, float2* spec,
+                                hipStream_t stream);
+hipError_t launch_x_inverse_any(const ShapePlan& sp, const ConvGeom& g, const float2* spec, const EpilogueArgs& e,
+                                hipStream_t stream, int nwg);
+
+// Register-resident kernels of a fixed length (fft_fast.hip).
 bool fast_size(int n);
+inline bool register_size(const FftPlan& p) { return fast_size(p.n) || any_size(p); }
 int x_fast_rows_per_wg(int M);
 hipError_t launch_y_fast(const ShapePlan& sp, float2* spec, int zlo, int zhi, int ylo, int yhi, float dir,
                          hipStream_t stream);
-// y pass whose input holds data only in rows [in_lo.y, in_hi.y) of planes
-// [in_lo.z, in_hi.z); every other input row is read as zero (register kernels).
 hipError_t launch_y_fast_window(const ShapePlan& sp, float2* spec, int zlo, int zhi, int ylo, int yhi, float dir,
                                 Int3 in_lo, Int3 in_hi, hipStream_t stream);
 hipError_t launch_z_fast(const ShapePlan& sp, float2* spec, const float2* kspec, float scale, int zlo, int zhi,
-                         hipStream_t stream, float dir, float2* aux = nullptr, const float2* pre = nullptr);
+                         hipStream_t stream, float dir, float2* aux, const float2* pre, const double* wsum, double kdc);
 hipError_t launch_z_fast_grad(const ShapePlan& sp, float2* spec, const float2* what, const float2* khat, float2* corr,
                               int mode, int first, Int3 shift, int zlo, int zhi, int kz, const double* rsum,
                               float2* adj, bool adj_add, hipStream_t stream);
@@ -346,11 +368,21 @@ struct PassDesc {
 };
 constexpr int kMaxParamBytes = 640;
 bool pass_is_fast(const PassDesc& d);
+bool pass_is_any(const PassDesc& d);
 // Fill the kernel parameter block of one item; returns its size in bytes and
 // the item's own grid (gx, gy); *lds = dynamic LDS bytes (generic) and
 // *cls = template selector (fast).
 int build_generic_params(const PassDesc& d, void* out, int* gx, int* gy, size_t* lds);
 int build_fast_params(const PassDesc& d, void* out, int* gx, int* gy, int* cls);
+int build_any_params(const PassDesc& d, void* out, int* gx, int* gy, int* cls, int* threads, size_t* lds);
+int build_any_x_params(const PassDesc& d, void* out, int* gx, int* gy, int* cls, int* threads, size_t* lds);
+int build_any_yz_params(const PassDesc& d, void* out, int* gx, int* gy, int* cls, int* threads, size_t* lds);
+hipError_t launch_batch_any(int kind, int cls, int epi, const void* items, const int* prefix, const int* gx, int nitems,
+                            int nwg, int threads, size_t lds, hipStream_t stream);
+hipError_t launch_batch_any_x(int kind, int cls, int epi, const void* items, const int* prefix, const int* gx,
+                              int nitems, int nwg, int threads, size_t lds, hipStream_t stream);
+hipError_t launch_batch_any_yz(int kind, int cls, const void* items, const int* prefix, const int* gx, int nitems,
+                               int nwg, int threads, size_t lds, hipStream_t stream);
 hipError_t launch_batch_generic(int kind, int epi, const void* items, const int* prefix, const int* gx, int nitems,
                                 int nwg, size_t lds, hipStream_t stream);
 // tasks (x and y forward only, optional): one (item, plane) per wpt
@@ -418,6 +450,9 @@ hipError_t launch_fold_gather(const float* win, Int3 wd, Int3 lo, Int3 n, float*
 hipError_t launch_reduce_sum(const double* part, int n, double* out, hipStream_t stream);
 // *out = sum of a[0, n) in double, through nparts partials in part.
 hipError_t launch_sum_to(const float* a, int64_t n, double* part, int nparts, double* out, hipStream_t stream);
+// *out = sum in double of the window [lo, lo + wd) of the mirror-extended image.
+hipError_t launch_window_sum_to(const float* img, Int3 n, Int3 lo, Int3 wd, double* part, int nparts, double* out,
+                                hipStream_t stream);
 // spec[0] = (float) *v (the zero-frequency value of a spectrum).
 hipError_t launch_set_dc(float2* spec, const double* v, hipStream_t stream);
 

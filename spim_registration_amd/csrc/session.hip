@@ -74,6 +74,13 @@ FftPlan make_plan(int n) {
   while (m % 2 == 0) push(2);
   while (m % 3 == 0) push(3);
   while (m % 5 == 0) push(5);
+  // two radices of the register kernels, as close to each other as they come:
+  // the pass with fewer butterflies leaves threads idle, and a kernel's
+  // registers grow with its larger radix
+  static const int radices[] = {2, 3, 4, 5, 6, 8, 9, 10, 12, 15, 16, 18, 20, 24, 25, 27, 30, 32};
+  for (int a : radices)
+    for (int b : radices)
+      if (a * b == n && a >= b && (!p.a || a < p.a)) p.a = a, p.b = b;
   return p;
 }
 
@@ -388,7 +395,10 @@ namespace mvd {
 // that share the kernel class; items, prefix and per-item grids live on the device.
 struct PassLaunch {
   int kind = 0, cls = 0, epi = 0, nitems = 0, nwg = 0;
-  int path = 0;    // 0 generic kernels, 1 register-resident kernels, 2 fused x-y kernels
+  // 0 LDS kernels, 1 register kernels of a fixed length, 2 fused x-y kernels,
+  // 3 register kernels of any length
+  int path = 0;
+  int threads = 0;  // per workgroup (path 3)
   int timing = 0;  // TimingClass of the launch
   bool lines = false;  // z pass with one kernel spectrum for all items: grid (lx, ly) of lines
   int lx = 0, ly = 0;
@@ -673,6 +683,7 @@ struct mvd_session {
     const ShapePlan* plan = nullptr;
     std::vector<ConvGeom> blocks;
     DeviceBuf k1hat, k2hat;
+    double k1dc = 0.0;  // zero-frequency value of k1hat before its rounding
     int nwg_update = 0;
   };
   std::vector<View> views;
@@ -683,6 +694,7 @@ struct mvd_session {
   DeviceBuf g_spec_a, g_spec_b, g_spec_c, g_spec_d, g_box, g_khat, g_psi, g_part_sum, g_part_max;
   DeviceBuf g_adj;  // the views' adjoint spectra summed (views sharing one window)
   DeviceBuf g_out;  // per call: the views' NLL sums (double) and PSF gradients (float), copied out at once
+  DeviceBuf g_wsum;  // the double sum of the window of W^, and its partials
   DeviceBuf g_rsum;  // partials and the double sum of one block's residual
   DeviceBuf g_crop, g_gpsi;
   bool g_gpsi_ready = false;
@@ -756,6 +768,11 @@ int build_pass_launches(const std::vector<PassDesc>& descs, std::vector<PassLaun
     } else if (pass_is_fast(d)) {
       path = 1;
       build_fast_params(d, tmp, &gx, &gy, &cls);
+    } else if (pass_is_any(d)) {
+      int nt;
+      size_t lds;
+      path = 3;
+      build_any_params(d, tmp, &gx, &gy, &cls, &nt, &lds);
     }
     // (the 384-point lines kernel exists with plane tables only: without them
     // it needs more than 256 VGPRs; those items take the batched z kernel)
@@ -776,16 +793,18 @@ int build_pass_launches(const std::vector<PassDesc>& descs, std::vector<PassLaun
     std::vector<int> prefix(1, 0), gxs;
     for (const PassDesc* d : kv.second) {
       unsigned char tmp[kMaxParamBytes];
-      int gx = 0, gy = 0, cls = 0;
+      int gx = 0, gy = 0, cls = 0, threads = 0;
       size_t lds = 0;
       const int n = L.path == 2   ? build_xy_params(*d, tmp, &gx, &gy, &cls)
                     : L.path == 1 ? build_fast_params(*d, tmp, &gx, &gy, &cls)
+                    : L.path == 3 ? build_any_params(*d, tmp, &gx, &gy, &cls, &threads, &lds)
                                   : build_generic_params(*d, tmp, &gx, &gy, &lds);
       MVD_REQUIRE(n > 0 && n <= kMaxParamBytes, "internal: parameter block size");
       blob.insert(blob.end(), tmp, tmp + n);
       gxs.push_back(std::max(gx, 1));
       prefix.push_back(prefix.back() + gx * gy);
       L.lds = std::max(L.lds, lds);
+      L.threads = std::max(L.threads, threads);
     }
     L.nitems = (int)kv.second.size();
     L.nwg = prefix.back();
@@ -853,6 +872,9 @@ hipError_t enqueue_pass_launch(const PassLaunch& L, hipStream_t st) {
   if (L.path == 1)
     return launch_batch_fast(L.kind, L.cls, L.items.p, L.prefix.as<int>(), L.gx.as<int>(), L.nitems, L.nwg, st,
                              L.wpt ? L.ptasks.as<int2>() : nullptr, L.wpt);
+  if (L.path == 3)
+    return launch_batch_any(L.kind, L.cls, L.epi, L.items.p, L.prefix.as<int>(), L.gx.as<int>(), L.nitems, L.nwg,
+                            L.threads, L.lds, st);
   return launch_batch_generic(L.kind, L.epi, L.items.p, L.prefix.as<int>(), L.gx.as<int>(), L.nitems, L.nwg, L.lds,
                               st);
 }
@@ -1042,12 +1064,14 @@ int run_conv(mvd_session* s, const ShapePlan& sp, const ConvGeom& g, const float
 }
 
 // Spectrum of a kernel wrapped into the FFT box of sp, scaled by 1/(qx qy qz).
-int kernel_spectrum(mvd_session* s, const ShapePlan& sp, const std::vector<float>& k, Int3 kd, DeviceBuf* out) {
+// *dc (nullable): its zero-frequency value before the rounding to float.
+int kernel_spectrum(mvd_session* s, const ShapePlan& sp, const std::vector<float>& k, Int3 kd, DeviceBuf* out,
+                    double* dc_out = nullptr) {
   MVD_CHECK(out->ensure(sizeof(float2) * sp.spectrum_elems()));
-  // the generic x pass leaves the row padding [hx, pitch) unwritten; zeros
+  // the LDS x pass leaves the row padding [hx, pitch) unwritten; zeros
   // there keep the (discarded) padding lanes of the z pass finite.  The
-  // register x pass stores the padding as zeros with every row.
-  if (!fast_size(sp.q.x / 2))
+  // register x passes store the padding as zeros with every row.
+  if (!fast_size(sp.q.x / 2) && !any_size(sp.px))
     MVD_CHECK(hipMemsetAsync(out->p, 0, sizeof(float2) * sp.spectrum_elems(), s->stream));
   DeviceBuf dk;
   MVD_CHECK(dk.ensure(sizeof(float) * k.size()));
@@ -1077,6 +1101,7 @@ int kernel_spectrum(mvd_session* s, const ShapePlan& sp, const std::vector<float
   long double sum = 0.0L;
   for (float v : k) sum += v;
   const float2 dc = make_float2((float)(sum / n), 0.f);
+  if (dc_out) *dc_out = (double)(sum / n);
   MVD_CHECK(hipMemcpyAsync(out->p, &dc, sizeof(dc), hipMemcpyHostToDevice, s->stream));
   MVD_CHECK(hipStreamSynchronize(s->stream));
   return 0;
@@ -1363,7 +1388,7 @@ int build_geometry(mvd_session* s, int v) {
 
 int view_spectra(mvd_session* s, int v) {
   mvd_session::View& view = s->views[v];
-  int rc = kernel_spectrum(s, *view.plan, view.k1, view.kd, &view.k1hat);
+  int rc = kernel_spectrum(s, *view.plan, view.k1, view.kd, &view.k1hat, &view.k1dc);
   if (rc) return rc;
   return kernel_spectrum(s, *view.plan, view.k2, view.kd, &view.k2hat);
 }
@@ -1963,7 +1988,7 @@ int mvd_nll_grad_device(mvd_session* s, const float* psi, const float* const* ps
     // fuse_r (one block, register x and y passes): the pass-1 x inverse turns
     // the residual rows into their x transform in the window spectrum Cs and
     // sums them; the residual image is not written
-    const bool fuse_r = keep_w && fast_size(q.x / 2) && fast_size(q.y) && !xy_fused(sp);
+    const bool fuse_r = keep_w && register_size(sp.px) && register_size(sp.py) && !xy_fused(sp);
     // the summed correlation spectrum D: its own buffer unless one block's
     // correlation goes through B (keep_w, or the separate launches with one block)
     const bool own_d = z_grad ? !keep_w : blocks.size() > 1;
@@ -1979,10 +2004,12 @@ int mvd_nll_grad_device(mvd_session* s, const float* psi, const float* const* ps
     double* rsum = s->g_rsum.as<double>() + rparts;
     // the kernel spectrum: the prepared view's own when the PSF is its kernel1
     const float2* Kh = nullptr;
+    double Kdc = 0.0;
     if (s->prepared && view.plan == spp && view.k1hat.p && pk == view.k1) {
       Kh = view.k1hat.as<float2>();
+      Kdc = view.k1dc;
     } else {
-      int rc = kernel_spectrum(s, sp, pk, k, &s->g_khat);
+      int rc = kernel_spectrum(s, sp, pk, k, &s->g_khat, &Kdc);
       if (rc) return rc;
       Kh = s->g_khat.as<float2>();
     }
@@ -2007,11 +2034,17 @@ int mvd_nll_grad_device(mvd_session* s, const float* psi, const float* const* ps
         if (!(w_plan == spp && same_window(w_geom, g))) {
           MVD_CHECK(launch_xy_forward_passes(sp, g, psrc, kGatherMirror, A, st));
           MVD_CHECK(launch_z(sp, A, nullptr, 1.f, 0, q.z, st, -1.f));
+          MVD_CHECK(s->g_wsum.ensure(sizeof(double) * (kRsumParts + 1)));
+          MVD_CHECK(launch_window_sum_to(psrc, n, g.off, g.win, s->g_wsum.as<double>() + 1, kRsumParts,
+                                         s->g_wsum.as<double>(), st));
           w_plan = spp;
           w_geom = g;
         }
         const int zlo = g.eff_local.z, zhi = g.eff_local.z + g.eff_size.z;
-        MVD_CHECK(launch_z(sp, B, Kh, 1.f, zlo, zhi, st, -1.f, nullptr, A));
+        // W^(0) P^(0) from the double sums: an ulp of it scales every b, to
+        // which the PSF gradient responds about a thousand times more strongly
+        // than to the product's other values
+        MVD_CHECK(launch_z(sp, B, Kh, 1.f, zlo, zhi, st, -1.f, nullptr, A, s->g_wsum.as<double>(), Kdc));
         if (fuse_r) {
           e.rspec = s->g_spec_c.as<float2>();
           e.rpitch = sp.pitch;
@@ -2051,7 +2084,7 @@ int mvd_nll_grad_device(mvd_session* s, const float* psi, const float* const* ps
         // effective box are read as zero by the y pass
         const Int3 lo = g.eff_local;
         const Int3 hi = {lo.x + g.eff_size.x, lo.y + g.eff_size.y, lo.z + g.eff_size.z};
-        MVD_CHECK(launch_y_fast_window(sp, Cs, 0, q.z, 0, q.y, -1.f, lo, hi, st));
+        MVD_CHECK(launch_y_window(sp, Cs, 0, q.z, 0, q.y, -1.f, lo, hi, st));
       } else {
         // R^ = FFT(residual of this block's effective region, zero elsewhere in
         // the window); the residual image itself when that region is the image
