@@ -69,6 +69,19 @@ def kernel_bytes(geom_blocks, q, img_n):
     return b
 
 
+def row_kernel_bytes(size_xyz, k_xyz):
+    """The same for the whole-image iteration by rows, without padding: the y
+    passes between one x-transformed row per image row and the window's rows,
+    the z pass over the window with its kernel spectrum, the x pass from row to
+    row with the epilogue."""
+    (nx, ny, nz), (kx, ky, kz) = size_xyz, k_xyz
+    hx, wy, wz = (nx + kx - 1) // 2 + 1, ny + ky - 1, nz + kz - 1
+    rows, E = 8 * hx * ny * nz, nx * ny * nz
+    return dict(y_forward=2 * (rows + 8 * hx * wy * nz), z_conv=2 * 8 * hx * wy * (2 * nz + wz),
+                y_inverse=2 * (rows + 8 * hx * wy * nz), x_inverse_quotient=2 * rows + 4 * E,
+                x_inverse_update=2 * rows + 12 * E)
+
+
 def path_bytes(geom_blocks, q):
     qx, qy, qz = q
     P = qx * qy * qz
@@ -792,6 +805,11 @@ def main():
     q = geo["fft"]
     effs = block_effective_sizes(w["size_xyz"], w["k_xyz"], blk) if blk else [tuple(w["size_xyz"])]
     kb = kernel_bytes(effs, q, n)
+    # by rows the forward x pass runs once per call, not once per convolution
+    by_rows = max(tim.get(c, (0, 0))[1] for c in ("x_forward", "xy_forward")) < nv * timed_iters
+    if by_rows:
+        kb = row_kernel_bytes(w["size_xyz"], w["k_xyz"])
+        win = [a + b - 1 for a, b in zip(w["size_xyz"], w["k_xyz"])]
     per_class = {}
     for name, (ms, cnt) in tim.items():
         if cnt and name in kb:
@@ -808,7 +826,7 @@ def main():
             traffic = json.load(open(tfile)).get(dom)
         except Exception:
             traffic = None
-    pb = path_bytes(effs, q) * nv * args.steps
+    pb = (path_bytes([tuple(w["size_xyz"])], win) if by_rows else path_bytes(effs, q)) * nv * args.steps
     path_gbs = pb / sec / 1e9
     log("per-kernel: " + json.dumps(per_class, indent=None))
 
@@ -875,7 +893,8 @@ def main():
                      "avg_launch_us": round(dc["avg_us"], 2)},
         "path_roofline": {"achieved": round(path_gbs, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                           "frac": round(path_gbs / HBM_PEAK_GBS, 4),
-                          "model": "8P + 48H + 20E bytes per block, view and iteration"},
+                          "model": "8P + 48H + 20E bytes per view and iteration, P and H of the window image + K - 1"
+                          if by_rows else "8P + 48H + 20E bytes per block, view and iteration"},
         "copy_probe": {"GB/s": round(copy_gbs, 1), "what": "torch device-to-device copy of 1 GiB (read + write)"},
         "kernels": {k: {"avg_us": round(v["avg_us"], 2), "GB/s": round(v["gbs"], 1),
                         "share": round(v["ms_total"] / sum(x["ms_total"] for x in per_class.values()), 3)}

@@ -156,7 +156,13 @@ int mvd_extract_psf(int device, const float* img, int nx, int ny, int nz, const 
  * model (ExtractPSF.transformPSF, deconv/ExtractPSF.java:325-372). */
 int mvd_psf_transform_size(const int* psf_size, const double* model, int* new_size);
 
-/* FFT shape of each block window (call before mvd_prepare). */
+/* FFT shape of each block window (call before mvd_prepare).  The iteration of a
+ * session whose views have kernels of one size runs over the whole image by
+ * rows in a shape of its own, whatever the blocks (blocked and whole
+ * convolutions are one operator; only rounding differs); the gradient, and
+ * sessions that it does not take (kernels of several sizes, arrays of 4 GiB or
+ * more, buffers past half of the free memory), use the block windows.
+ * mvd_get_geometry reports the block windows. */
 enum {
   MVD_FFT_SMOOTH = 0,   /* smallest 5-smooth size per axis (default) */
   MVD_FFT_POW2 = 1,     /* smallest power of two per axis (up to 1024) */

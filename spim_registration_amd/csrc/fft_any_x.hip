@@ -19,8 +19,10 @@ struct RowGroup {
 RowGroup row_group_of(const FftPlan& p) {
   const AnyFft f = any_fft(p);
   RowGroup g;
-  const int ex = f.b * f.pa;
-  g.slots = (ex > p.n + 1 ? ex : p.n + 1) | 1;
+  // rows start a slots apart modulo the 32 slots of a full set of banks, so that
+  // the second pass's loads (a neighbouring slots of each row) run through them
+  const int ex = f.b * f.pa, least = ex > p.n + 1 ? ex : p.n + 1;
+  g.slots = least + ((p.a - least) % 32 + 32) % 32;
   g.rows = 256 / p.a;
   while (g.rows > 1 && sizeof(float2) * (2 * p.n + (size_t)g.rows * g.slots) > 64 * 1024) --g.rows;
   g.nt = (g.rows * p.a + 63) / 64 * 64;
@@ -248,25 +250,25 @@ __device__ __forceinline__ void x_any_inverse_body(const XAnyInvParams& P, int b
   const double inv_lambda = rl_inv_lambda(e.lambda);
   double my_sum = 0.0, my_rsum = 0.0;
   float my_max = -1.f;
-  const bool r_rows = EPI == kEpiResidual && e.rspec != nullptr;
+  const bool r_rows = EPI != kEpiStore && e.rspec != nullptr;
   // A wave takes whole rows in pieces of 64 voxels; the inputs of four pieces
   // are loaded before the first is computed (piece by piece, the memory
   // latency of each would follow on the one before).
   constexpr int U = 4;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int live_rows = min(P.rows, nrows - row0), pieces = (nx + 63) >> 6;
-  int l = wave, c = 0;
+  const int live_rows = min(P.rows, nrows - row0);
+  int l = wave, x0 = 0;
+  // the row's place in the destination (wave-uniform, one division in all);
+  // images hold fewer than 2^31 voxels (checked by the host)
+  int zo = (row0 + l) / ny, yo = row0 + l - zo * ny;
   while (l < live_rows) {
     int base[U], vofs[U];
     bool on[U];
     float in0[U], in1[U], in2[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const int x = c * 64 + lane;
+      const int x = x0 + lane;
       on[u] = l < live_rows && x < nx;
-      const int row = row0 + min(l, live_rows - 1);
-      const int zo = row / ny, yo = row - zo * ny;
-      // images hold fewer than 2^31 voxels (checked by the host)
       base[u] = g.eff_offset.x + g.dst.x * ((g.eff_offset.y + yo) + g.dst.y * (g.eff_offset.z + zo)) + x;
       vofs[u] = 2 * l * P.slots + g.eff_local.x + x;
       in0[u] = in2[u] = 0.f;
@@ -278,9 +280,11 @@ __device__ __forceinline__ void x_any_inverse_body(const XAnyInvParams& P, int b
         if (EPI == kEpiUpdate && e.weight_mode != kWeightNone) in1[u] = gmem(e.weight)[base[u]];
         if (EPI == kEpiUpdate && e.weight_mode == kWeightVirtual) in2[u] = gmem(e.wsum)[base[u]];
       }
-      if (++c == pieces) {
-        c = 0;
+      x0 += 64;
+      if (x0 >= nx) {
+        x0 = 0;
         l += nw;
+        for (yo += nw; yo >= ny; yo -= ny) ++zo;
       }
     }
 #pragma unroll
@@ -291,7 +295,9 @@ __device__ __forceinline__ void x_any_inverse_body(const XAnyInvParams& P, int b
       if (EPI == kEpiStore) {
         *dst = val;
       } else if (EPI == kEpiQuotient) {
-        *dst = rl_quotient(val, in0[u]);
+        const float ratio = rl_quotient(val, in0[u]);
+        if (r_rows) fbuf[vofs[u]] = ratio;
+        else *dst = ratio;
       } else if (EPI == kEpiResidual) {
         float rv = 0.f;
         if (val > 0.f) {
@@ -309,6 +315,7 @@ __device__ __forceinline__ void x_any_inverse_body(const XAnyInvParams& P, int b
         if (e.weight_mode == kWeightVirtual) w = (float)java_min(1.0, (double)w / (double)in2[u] * e.osem);
         const float next = rl_next_value(in0[u], val, w, e.lambda, inv_lambda);
         *dst = next;
+        if (r_rows) fbuf[vofs[u]] = next;
         const float change = fabsf(next - in0[u]);
         my_sum += (double)change;
         my_max = java_maxf(my_max, change);
@@ -316,10 +323,19 @@ __device__ __forceinline__ void x_any_inverse_body(const XAnyInvParams& P, int b
     }
   }
   if (r_rows) {
-    // the window rows: the effective row at eff_local, zeros elsewhere
-    for (int r = wave; r < live_rows; r += nw)
-      for (int x = lane; x < 2 * M; x += 64)
-        if (x < g.eff_local.x || x >= g.eff_local.x + nx) fbuf[2 * r * P.slots + x] = 0.f;
+    // the window rows: the effective row at eff_local; outside it the residual
+    // is zero, the ratio one and the estimate mirrored, up to the window's end
+    if (EPI == kEpiUpdate) __syncthreads();
+    for (int r = wave; r < live_rows; r += nw) {
+      float* wrow = fbuf + 2 * r * P.slots;
+      for (int h = lane; h < 2 * M - nx; h += 64) {  // the row's positions outside the image
+        const int x = h < g.eff_local.x ? h : h + nx, p = x - g.eff_local.x;
+        float v = 0.f;
+        if (EPI == kEpiQuotient && x < g.win.x) v = 1.f;
+        if (EPI == kEpiUpdate && x < g.win.x) v = wrow[g.eff_local.x + mirror_single(p, nx)];
+        wrow[x] = v;
+      }
+    }
   }
   if (EPI == kEpiUpdate || EPI == kEpiResidual) {
     for (int o = 32; o > 0; o >>= 1) {
@@ -343,12 +359,12 @@ __device__ __forceinline__ void x_any_inverse_body(const XAnyInvParams& P, int b
       }
       gmem(e.part_sum)[bx] = s;
       gmem(e.part_max)[bx] = m;
-      if (r_rows) gmem(e.part_rsum)[bx] = rs;
+      if (EPI == kEpiResidual && r_rows) gmem(e.part_rsum)[bx] = rs;
     }
   }
-  if constexpr (EPI == kEpiResidual) {
+  if constexpr (EPI != kEpiStore) {
     if (!r_rows) return;  // uniform
-    // the x transform of the residual rows into the residual's window spectrum
+    // the x transform of the window rows
     const int l = (int)__umulhi((unsigned)threadIdx.x, f.mb), j = threadIdx.x - l * f.b;
     __syncthreads();
     with_radix_a<RC>(f.a, [&](auto rc) {
@@ -461,7 +477,7 @@ int build_any_x_params(const PassDesc& d, void* out, int* gx, int* gy, int* cls,
     return sizeof(P);
   }
   const XAnyInvParams P{d.g, d.spec, d.e, sp.tw_x, any_fft(sp.px), sp.pitch, r.rows, r.slots};
-  *gx = x_inverse_workgroups(sp, d.g);
+  *gx = (d.g.eff_size.y * d.g.eff_size.z + r.rows - 1) / r.rows;
   *cls = any_class(sp.px);
   std::memcpy(out, &P, sizeof(P));
   return sizeof(P);

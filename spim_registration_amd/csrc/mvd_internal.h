@@ -220,10 +220,13 @@ struct EpilogueArgs {
   double* part_sum;      // per-workgroup statistics of the update
   float* part_max;
   float wconst = 1.f;    // the weight of every voxel under kWeightNone
-  // kEpiResidual, register x inverse only: instead of storing the residual,
-  // transform its rows (the block's effective box placed in its window, zeros
-  // elsewhere) along x into rspec (window rows, pitch rpitch) and write each
-  // workgroup's residual sum (double) to part_rsum
+  // register x inverse only: the rows of the result go on to their transform
+  // along x, into rspec (window rows, pitch rpitch).  kEpiResidual: instead of
+  // storing the residual, the block's effective box placed in its window with
+  // zeros elsewhere; each workgroup's residual sum (double) to part_rsum.
+  // kEpiQuotient (two-radix kernels): instead of storing the ratio, with ones
+  // outside it.  kEpiUpdate (two-radix kernels): the new estimate, mirrored
+  // outside it, besides storing it.
   float2* rspec = nullptr;
   int rpitch = 0;
   double* part_rsum = nullptr;
@@ -360,12 +363,37 @@ struct PassDesc {
   int zlo, zhi, ylo, yhi;
   float dir, scale;
   int xy;  // x passes of a fused x-y item (no separate y pass)
+  bool any = false;  // x passes: the two-radix kernels also where the length has its own
   // z pass in the lines kernel only: input planes through a table of plane
   // indices into the arena of spectra (nullptr: plane z of spec)
   const unsigned short* ztab = nullptr;
   const float2* arena = nullptr;
   unsigned arena_bytes = 0;
 };
+// y and z passes between x-transformed image rows and tiles of planes
+// (fft_rows.hip): kPassYForward, kPassYInverse (one tile) and kPassZConv (all
+// tiles of an image).
+struct RowsPass {
+  int kind;
+  const ShapePlan* sp;
+  Int3 n;                // image size
+  float2* rows;          // [n.z][n.y][pitch], then the x transform of a row of the constant outside the image
+  float2* planes;        // slabs of the tile (z: of all tiles, then of a plane of that constant)
+  const float2* kspec;
+  bool kslabs;           // kspec is stored in slabs (launch_to_slabs)
+  bool mirror;           // the image mirrored outside, else the constant
+  int off_y, win_y;      // image row of the tile's row 0; rows that hold its window
+  int lo_y, cnt_y, eoff_y;  // inverse: tile rows [lo, lo + cnt) are the image rows from eoff
+  int nplanes;
+  int off_z, win_z, tiles;  // the window's first plane is image plane -off_z
+};
+// Slabs of eight rows, [(q.y + 7) / 8][planes][8][pitch]: their size, and a
+// spectrum of a shape stored in them.
+int64_t slab_elems(const ShapePlan& sp, int planes);
+hipError_t launch_to_slabs(const ShapePlan& sp, const float2* in, float2* out, hipStream_t stream);
+int build_rows_params(const RowsPass& d, void* out, int* gx, int* gy, int* cls, int* threads, size_t* lds);
+hipError_t launch_rows(int kind, int cls, const void* items, const int* prefix, const int* gx, int nitems, int nwg,
+                       int threads, size_t lds, hipStream_t stream);
 constexpr int kMaxParamBytes = 640;
 bool pass_is_fast(const PassDesc& d);
 bool pass_is_any(const PassDesc& d);

@@ -391,20 +391,43 @@ static std::vector<float> inverted(const std::vector<float>& k, Int3 d) {
 
 namespace mvd {
 
+// The device tables of a list of launches (items, workgroup prefixes and grids)
+// in one allocation, filled by one copy: three of each per launch took 1.6 ms
+// of the first iteration of three small views.
+struct LaunchTables {
+  std::vector<unsigned char> host;
+  DeviceBuf dev;
+  size_t add(const void* p, size_t n) {
+    const size_t at = (host.size() + 15) / 16 * 16;
+    host.resize(at + n);
+    std::memcpy(host.data() + at, p, n);
+    return at;
+  }
+  hipError_t upload() {
+    if (host.empty()) return hipSuccess;
+    const hipError_t e = dev.ensure(host.size());
+    return e != hipSuccess ? e : hipMemcpy(dev.p, host.data(), host.size(), hipMemcpyHostToDevice);
+  }
+};
+
 // One launch of a pass over a group of items (blocks of one or many stacks)
 // that share the kernel class; items, prefix and per-item grids live on the device.
 struct PassLaunch {
   int kind = 0, cls = 0, epi = 0, nitems = 0, nwg = 0;
   // 0 LDS kernels, 1 register kernels of a fixed length, 2 fused x-y kernels,
-  // 3 register kernels of any length
+  // 3 register kernels of any length, 4 the y and z passes of RowConv
   int path = 0;
-  int threads = 0;  // per workgroup (path 3)
+  int threads = 0;  // per workgroup (paths 3 and 4)
   int timing = 0;  // TimingClass of the launch
   bool lines = false;  // z pass with one kernel spectrum for all items: grid (lx, ly) of lines
   int lx = 0, ly = 0;
   bool reduce = false;
   size_t lds = 0;
-  DeviceBuf items, prefix, gx;
+  const LaunchTables* tab = nullptr;  // uploaded before the launch
+  size_t items_at = 0, prefix_at = 0, gx_at = 0;
+  const void* items() const { return tab->dev.as<unsigned char>() + items_at; }
+  const int* prefix() const { return reinterpret_cast<const int*>(tab->dev.as<unsigned char>() + prefix_at); }
+  const int* gx() const { return reinterpret_cast<const int*>(tab->dev.as<unsigned char>() + gx_at); }
   DeviceBuf sched;  // fused forward: one PlaneTask per workgroup
   bool has_sched = false;
   int table = 0;  // lines z pass reading its input planes through tables (1: 32-bit, 2: 64-bit offsets)
@@ -433,6 +456,13 @@ static const bool g_grad_fused = [] {
 }();
 static const bool g_grad_keep_w = [] {
   const char* v = std::getenv("MVD_GRAD_KEEP_W");
+  return !(v && v[0] == '0');
+}();
+
+// MVD_ROW_CONV=0: the iteration convolves the blocks one window each
+// (comparisons).
+static const bool g_row_conv = [] {
+  const char* v = std::getenv("MVD_ROW_CONV");
   return !(v && v[0] == '0');
 }();
 
@@ -684,6 +714,8 @@ struct mvd_session {
     std::vector<ConvGeom> blocks;
     DeviceBuf k1hat, k2hat;
     double k1dc = 0.0;  // zero-frequency value of k1hat before its rounding
+    DeviceBuf r1hat, r2hat;   // spectra in the shape of the session's RowConv
+    bool hat_ready = false;   // k1hat holds kernel1 (with a RowConv of another shape: made when asked for)
     int nwg_update = 0;
   };
   std::vector<View> views;
@@ -706,10 +738,43 @@ struct mvd_session {
   // spectra do not fit (the per-block loop then reuses d_spec).
   struct BlockBatch {
     bool built = false, enabled = true;
+    LaunchTables tables;
     DeviceBuf arena;                 // the block spectra, one after another
     std::vector<DeviceBuf> ztab;     // z-pass plane tables, per view and convolution
     std::vector<std::vector<PassLaunch>> view;  // per view: convolve1 passes, then convolve2 passes
   } bb;
+
+  // The iteration over the whole image by rows.  `rows` holds one
+  // x-transformed row of the window per image row; per convolution the y pass
+  // transforms them into the planes of each y tile (the mirrored or constant
+  // rows outside the image are read from the rows they mirror or from one
+  // constant row), the z pass convolves, the y pass comes back, and the x pass
+  // transforms each row back, computes the quotient or the update and
+  // transforms the new row forward again, ready for the next convolution.
+  // Against block windows this stores no row or plane twice, pads the image
+  // once instead of every block, and takes one pass less per convolution; the
+  // ratio image never reaches memory.  Blocked and whole convolutions are one
+  // operator, so only rounding depends on it.  Ten iterations of 6 views of
+  // 512x512x256 in 256^3 blocks (18 windows, 4.5 times the image's voxels)
+  // 156 -> 112 ms, five of 3 views of 421x337x203 in 192^3 blocks 24.6 -> 15.2
+  // ms, of four 311x263x149 views in one window 18.7 -> 16.2 ms.  The y passes
+  // run at 5.5 to 5.9 TB/s; the z pass (3.5 TB/s) and the x pass (3.6) are held
+  // by VALU issue (55 %) and the latency of their three exchanges together.
+  struct RowConv {
+    bool on = false, shared = false, consts = false;  // shared: the views' own spectra have this shape
+    const ShapePlan* plan = nullptr;
+    Int3 kd{0, 0, 0}, win{0, 0, 0};
+    struct Tile {
+      int eoff, cnt;  // image rows [eoff, eoff + cnt)
+    };
+    std::vector<Tile> tiles;
+    int nwg = 0;  // workgroups of the x pass
+    // rows: an x-transformed row per image row, then one of the constant 1
+    // (what the ratio is outside the image); planes: the tiles', then one of it
+    DeviceBuf rows, planes;
+    DeviceBuf plain;  // a kernel spectrum before it goes to slabs
+    ConvGeom geom{};  // of the x pass: rows of the image
+  } rc;
 
   int fft_policy = MVD_FFT_SMOOTH;
   int psf_type = MVD_PSF_EFFICIENT_BAYESIAN;
@@ -745,7 +810,7 @@ int timing_class(int kind, int path, int epi) {
 // epilogue) -- and appends one launch per group.
 // fwd_tasks: the task list of the fused forward group when the caller planned
 // it (plan_conv_planes); otherwise forward_plane_tasks makes one.
-int build_pass_launches(const std::vector<PassDesc>& descs, std::vector<PassLaunch>* out,
+int build_pass_launches(const std::vector<PassDesc>& descs, LaunchTables* tab, std::vector<PassLaunch>* out,
                         const std::vector<PlaneTask>* fwd_tasks = nullptr,
                         const std::vector<int2>* plane_tasks = nullptr, bool wide = false) {
   // z items (register kernels) that share a kernel spectrum and shape with at
@@ -765,7 +830,7 @@ int build_pass_launches(const std::vector<PassDesc>& descs, std::vector<PassLaun
     if (d.xy) {
       path = 2;
       build_xy_params(d, tmp, &gx, &gy, &cls);
-    } else if (pass_is_fast(d)) {
+    } else if (!d.any && pass_is_fast(d)) {
       path = 1;
       build_fast_params(d, tmp, &gx, &gy, &cls);
     } else if (pass_is_any(d)) {
@@ -823,12 +888,10 @@ int build_pass_launches(const std::vector<PassDesc>& descs, std::vector<PassLaun
       for (const PassDesc* d : kv.second)
         MVD_REQUIRE(specs.insert(d->spec).second, "internal: z items of one launch share a spectrum");
     }
-    MVD_CHECK(L.items.ensure(blob.size()));
-    MVD_CHECK(hipMemcpy(L.items.p, blob.data(), blob.size(), hipMemcpyHostToDevice));
-    MVD_CHECK(L.prefix.ensure(sizeof(int) * prefix.size()));
-    MVD_CHECK(hipMemcpy(L.prefix.p, prefix.data(), sizeof(int) * prefix.size(), hipMemcpyHostToDevice));
-    MVD_CHECK(L.gx.ensure(sizeof(int) * gxs.size()));
-    MVD_CHECK(hipMemcpy(L.gx.p, gxs.data(), sizeof(int) * gxs.size(), hipMemcpyHostToDevice));
+    L.tab = tab;
+    L.items_at = tab->add(blob.data(), blob.size());
+    L.prefix_at = tab->add(prefix.data(), sizeof(int) * prefix.size());
+    L.gx_at = tab->add(gxs.data(), sizeof(int) * gxs.size());
     if (L.path == 2 && L.kind == kPassXForward && g_xcd_schedule) {
       const std::vector<PlaneTask> tasks = fwd_tasks ? *fwd_tasks : forward_plane_tasks(kv.second, g_plane_dedup);
       size_t stores = 0;
@@ -863,20 +926,92 @@ int build_pass_launches(const std::vector<PassDesc>& descs, std::vector<PassLaun
   return 0;
 }
 
+// One launch per kernel class of the y or z passes of RowConv items.
+int build_rows_launches(const std::vector<RowsPass>& passes, LaunchTables* tab, std::vector<PassLaunch>* out) {
+  std::map<std::pair<int, int>, std::vector<const RowsPass*>> groups;
+  unsigned char tmp[kMaxParamBytes];
+  for (auto& d : passes) {
+    int gx, gy, cls, threads;
+    size_t lds;
+    build_rows_params(d, tmp, &gx, &gy, &cls, &threads, &lds);
+    // a launch gives every workgroup the LDS of its largest item: items that fit
+    // four, three or two workgroups per CU go separately
+    const int share = lds <= 40 * 1024 ? 0 : lds <= 53 * 1024 ? 1 : 2;
+    groups[{cls, share}].push_back(&d);
+  }
+  for (auto& kv : groups) {
+    PassLaunch L;
+    L.kind = kv.second.front()->kind;
+    L.path = 4;
+    L.cls = kv.first.first;
+    L.timing = timing_class(L.kind, L.path, 0);
+    std::vector<unsigned char> blob;
+    std::vector<int> prefix(1, 0), gxs;
+    for (const RowsPass* d : kv.second) {
+      int gx, gy, cls, threads;
+      size_t lds;
+      const int n = build_rows_params(*d, tmp, &gx, &gy, &cls, &threads, &lds);
+      MVD_REQUIRE(n > 0 && n <= kMaxParamBytes, "internal: parameter block size");
+      blob.insert(blob.end(), tmp, tmp + n);
+      gxs.push_back(gx);
+      prefix.push_back(prefix.back() + gx * gy);
+      L.threads = std::max(L.threads, threads);
+      L.lds = std::max(L.lds, lds);
+    }
+    L.nitems = (int)kv.second.size();
+    L.nwg = prefix.back();
+    L.tab = tab;
+    L.items_at = tab->add(blob.data(), blob.size());
+    L.prefix_at = tab->add(prefix.data(), sizeof(int) * prefix.size());
+    L.gx_at = tab->add(gxs.data(), sizeof(int) * gxs.size());
+    out->push_back(std::move(L));
+  }
+  return 0;
+}
+
 hipError_t enqueue_pass_launch(const PassLaunch& L, hipStream_t st) {
-  if (L.reduce) return launch_reduce_stats_batch(L.items.as<ReduceItem>(), L.nitems, st);
-  if (L.lines) return launch_z_lines(L.cls, L.items.p, L.nitems, L.lx, L.ly, st, L.table);
+  if (L.reduce) return launch_reduce_stats_batch(static_cast<const ReduceItem*>(L.items()), L.nitems, st);
+  if (L.lines) return launch_z_lines(L.cls, L.items(), L.nitems, L.lx, L.ly, st, L.table);
   if (L.path == 2)
-    return launch_batch_xy(L.kind, L.cls, L.items.p, L.prefix.as<int>(), L.gx.as<int>(), L.nitems, L.nwg, st,
+    return launch_batch_xy(L.kind, L.cls, L.items(), L.prefix(), L.gx(), L.nitems, L.nwg, st,
                            L.has_sched ? L.sched.as<PlaneTask>() : nullptr);
   if (L.path == 1)
-    return launch_batch_fast(L.kind, L.cls, L.items.p, L.prefix.as<int>(), L.gx.as<int>(), L.nitems, L.nwg, st,
+    return launch_batch_fast(L.kind, L.cls, L.items(), L.prefix(), L.gx(), L.nitems, L.nwg, st,
                              L.wpt ? L.ptasks.as<int2>() : nullptr, L.wpt);
+  if (L.path == 4)
+    return launch_rows(L.kind, L.cls, L.items(), L.prefix(), L.gx(), L.nitems, L.nwg, L.threads, L.lds,
+                       st);
   if (L.path == 3)
-    return launch_batch_any(L.kind, L.cls, L.epi, L.items.p, L.prefix.as<int>(), L.gx.as<int>(), L.nitems, L.nwg,
+    return launch_batch_any(L.kind, L.cls, L.epi, L.items(), L.prefix(), L.gx(), L.nitems, L.nwg,
                             L.threads, L.lds, st);
-  return launch_batch_generic(L.kind, L.epi, L.items.p, L.prefix.as<int>(), L.gx.as<int>(), L.nitems, L.nwg, L.lds,
+  return launch_batch_generic(L.kind, L.epi, L.items(), L.prefix(), L.gx(), L.nitems, L.nwg, L.lds,
                               st);
+}
+
+// The epilogue of convolve1 (conv 0: psi -> ratio, quotient) or convolve2
+// (conv 1: ratio -> psi, update with statistics partials from `off`) of view v.
+EpilogueArgs conv_epilogue(mvd_session* s, int v, int conv, int off) {
+  const int wm = s->weight_mode == MVD_WEIGHTS_NONE ? kWeightNone
+                 : s->weight_mode == MVD_WEIGHTS_VIRTUAL ? kWeightVirtual
+                                                         : kWeightArray;
+  EpilogueArgs e{};
+  if (conv == 0) {
+    e.mode = kEpiQuotient;
+    e.dst = s->d_ratio.as<float>();
+    e.img = s->d_views.as<float>() + v * s->n;
+    return e;
+  }
+  e.mode = kEpiUpdate;
+  e.dst = s->d_psi.as<float>();
+  e.weight_mode = wm;
+  e.weight = wm == kWeightNone ? nullptr : s->d_weights.as<float>() + v * s->n;
+  e.wsum = s->d_wsum.as<float>();
+  e.osem = s->osem;
+  e.wconst = s->wconst;
+  e.lambda = s->lambda;
+  e.part_sum = s->d_part_sum.as<double>() + off;
+  e.part_max = s->d_part_max.as<float>() + off;
+  return e;
 }
 
 // The pass items of one convolution of view v over all its blocks: convolve1
@@ -885,9 +1020,6 @@ hipError_t enqueue_pass_launch(const PassLaunch& L, hipStream_t st) {
 void conv_pass_descs(mvd_session* s, int v, int conv, const std::vector<float2*>& spec,
                      std::vector<PassDesc> (&pass)[5]) {
   auto& view = s->views[v];
-  const int wm = s->weight_mode == MVD_WEIGHTS_NONE ? kWeightNone
-                 : s->weight_mode == MVD_WEIGHTS_VIRTUAL ? kWeightVirtual
-                                                         : kWeightArray;
   int off = 0;
   for (size_t bi = 0; bi < view.blocks.size(); ++bi) {
     const ConvGeom& g = view.blocks[bi];
@@ -929,25 +1061,197 @@ void conv_pass_descs(mvd_session* s, int v, int conv, const std::vector<float2*>
     PassDesc xi = d;
     xi.kind = kPassXInverse;
     xi.xy = fused;
-    if (conv == 0) {
-      xi.e.mode = kEpiQuotient;
-      xi.e.dst = s->d_ratio.as<float>();
-      xi.e.img = s->d_views.as<float>() + v * s->n;
-    } else {
-      xi.e.mode = kEpiUpdate;
-      xi.e.dst = s->d_psi.as<float>();
-      xi.e.weight_mode = wm;
-      xi.e.weight = wm == kWeightNone ? nullptr : s->d_weights.as<float>() + v * s->n;
-      xi.e.wsum = s->d_wsum.as<float>();
-      xi.e.osem = s->osem;
-      xi.e.wconst = s->wconst;
-      xi.e.lambda = s->lambda;
-      xi.e.part_sum = s->d_part_sum.as<double>() + off;
-      xi.e.part_max = s->d_part_max.as<float>() + off;
-      off += conv_inverse_workgroups(*view.plan, g);
-    }
+    xi.e = conv_epilogue(s, v, conv, off);
+    if (conv == 1) off += conv_inverse_workgroups(*view.plan, g);
     pass[4].push_back(xi);
   }
+}
+
+// How much work a pass of length n costs per value, relative to a short
+// length: the kernels of the larger radix classes hold fewer waves (class 3
+// half of class 1), a first pass with few butterflies idles threads, and
+// column passes whose line sets do not fit 80 KB sixteen columns wide read
+// half lines.  0: no two-radix kernel.
+double rows_length_cost(int n, bool columns) {
+  const FftPlan p = make_plan(n);
+  if (!any_size(p)) return 0.0;
+  const double by_class = p.a <= 16 ? 1.0 : p.a <= 20 ? 1.05 : p.a <= 27 ? 1.2 : 1.6;
+  const double split = 1.0 + 0.05 * ((double)p.a / p.b - 1.0);
+  return by_class * split * (columns && n > 576 ? 1.25 : 1.0);
+}
+
+// Cheapest length of at least w (0: none).
+int rows_length(int w, int most, bool columns, double* cost) {
+  int best = 0;
+  for (int n = std::max(w, 4); n <= most && n <= w + w / 2 + 8; ++n) {
+    const double c = fft_size_supported(n) ? n * rows_length_cost(n, columns) : 0.0;
+    if (c > 0.0 && (!best || c < *cost)) best = n, *cost = c;
+  }
+  return best;
+}
+
+// Chooses the whole-image iteration of a prepared session (RowConv): needs one
+// kernel size for all views (they share the rows), lengths with two-radix
+// kernels, and its buffers in half of the free memory; otherwise the blocks are
+// convolved one window each.  x and z are one window each, y as many tiles as
+// make the transforms cheapest.  The window of an unsplit view is kept when it
+// is about as cheap (within 10 %), so that the gradient uses the same spectra.
+int plan_rows(mvd_session* s) {
+  auto& r = s->rc;
+  r.on = r.consts = false;
+  if (!g_row_conv) return 0;
+  const Int3 n = s->img, kd = s->views[0].kd;
+  for (auto& v : s->views)
+    if (v.kd.x != kd.x || v.kd.y != kd.y || v.kd.z != kd.z) return 0;
+  const Int3 win = {n.x + kd.x - 1, n.y + kd.y - 1, n.z + kd.z - 1};
+  double cx = 0, cy = 0, cz = 0;
+  Int3 q;
+  q.x = 2 * rows_length((win.x + 1) / 2, 1024, false, &cx);
+  q.z = rows_length(win.z, 1024, true, &cz);
+  q.y = 0;
+  int tiles = 1;
+  for (int t = 1; t <= 64 && (t == 1 || t <= n.y / 32); ++t) {
+    double c = 0;
+    const int len = rows_length((n.y + t - 1) / t + kd.y - 1, 1024, true, &c);
+    // the z pass runs over the tiles' rows whatever their length
+    const double all = t * (0.4 * c + 0.6 * len);
+    if (len && (!q.y || all < cy)) {
+      q.y = len;
+      tiles = t;
+      cy = all;
+    }
+  }
+  if (q.x < 4 || !q.y || !q.z) return 0;
+  r.shared = false;
+  const auto& v0 = s->views[0];
+  if (v0.blocks.size() == 1 && any_size(v0.plan->px) && any_size(v0.plan->py) && any_size(v0.plan->pz)) {
+    const Int3 p = v0.plan->q;
+    const double c = (p.x / 2) * rows_length_cost(p.x / 2, false) * p.y * (0.4 * rows_length_cost(p.y, true) + 0.6) *
+                     p.z * rows_length_cost(p.z, true);
+    if (c <= 1.1 * cx * cy * cz) {
+      q = p;
+      tiles = 1;
+      r.shared = true;
+    }
+  }
+  r.plan = s->plans.get(q);
+  if (!r.plan) return -1;
+  const size_t row_bytes = sizeof(float2) * (size_t)r.plan->pitch;
+  const size_t rows_b = row_bytes * ((size_t)n.y * n.z + 1);
+  const size_t planes_b = sizeof(float2) * (size_t)(tiles * slab_elems(*r.plan, n.z) + slab_elems(*r.plan, 1));
+  const size_t spec_b = sizeof(float2) * (size_t)slab_elems(*r.plan, q.z);
+  if (std::max({rows_b, planes_b, spec_b}) >= (size_t(1) << 32)) return 0;  // 32-bit offsets
+  size_t need = rows_b + planes_b;
+  if (!r.shared) need += (2 * s->nviews + 1) * spec_b;
+  size_t have = r.rows.bytes + r.planes.bytes + r.plain.bytes, free_b = 0, total_b = 0;
+  for (auto& v : s->views) have += v.r1hat.bytes + v.r2hat.bytes;
+  MVD_CHECK(hipMemGetInfo(&free_b, &total_b));
+  if (need > have + free_b / 2) return 0;
+  r.kd = kd;
+  r.win = win;
+  r.tiles.clear();
+  const int eff = (n.y + tiles - 1) / tiles;
+  for (int y = 0; y < n.y; y += eff) r.tiles.push_back({y, std::min(eff, n.y - y)});
+  ConvGeom g{};
+  g.src = g.dst = g.eff_size = n;
+  g.off = {-(kd.x / 2), 0, 0};
+  g.win = {win.x, n.y, n.z};
+  g.q = {q.x, n.y, n.z};
+  g.eff_local = {kd.x / 2, 0, 0};
+  r.geom = g;
+  const int per = x_any_rows_per_wg(r.plan->px);
+  r.nwg = (n.y * n.z + per - 1) / per;
+  r.on = true;
+  return 0;
+}
+
+// The y and z passes and the x pass of one convolution of view v by rows.
+void rows_pass_descs(mvd_session* s, int v, int conv, std::vector<RowsPass> (&pass)[3], std::vector<PassDesc>* xinv) {
+  auto& r = s->rc;
+  auto& view = s->views[v];
+  const int64_t tile_elems = slab_elems(*r.plan, s->img.z);
+  RowsPass d{};
+  d.sp = r.plan;
+  d.n = s->img;
+  d.rows = r.rows.as<float2>();
+  d.mirror = conv == 0;
+  d.nplanes = s->img.z;
+  for (size_t t = 0; t < r.tiles.size(); ++t) {
+    RowsPass y = d;
+    y.planes = r.planes.as<float2>() + t * tile_elems;
+    y.off_y = r.tiles[t].eoff - r.kd.y / 2;
+    y.win_y = r.tiles[t].cnt + r.kd.y - 1;
+    y.lo_y = r.kd.y / 2;
+    y.cnt_y = r.tiles[t].cnt;
+    y.eoff_y = r.tiles[t].eoff;
+    y.kind = kPassYForward;
+    pass[0].push_back(y);
+    y.kind = kPassYInverse;
+    pass[2].push_back(y);
+  }
+  RowsPass z = d;
+  z.kind = kPassZConv;
+  z.planes = r.planes.as<float2>();
+  z.kspec = r.shared ? (conv == 0 ? view.k1hat : view.k2hat).as<float2>()
+                     : (conv == 0 ? view.r1hat : view.r2hat).as<float2>();
+  z.kslabs = !r.shared;
+  z.off_z = r.kd.z / 2;
+  z.win_z = r.win.z;
+  z.tiles = (int)r.tiles.size();
+  pass[1].push_back(z);
+  PassDesc x{};
+  x.kind = kPassXInverse;
+  x.any = true;
+  x.sp = r.plan;
+  x.g = r.geom;
+  x.spec = r.rows.as<float2>();
+  x.e = conv_epilogue(s, v, conv, 0);
+  x.e.rspec = r.rows.as<float2>();
+  x.e.rpitch = r.plan->pitch;
+  xinv->push_back(x);
+}
+
+// Buffers of the iteration by rows, and the spectra of the constant one that
+// the ratio has outside the image: a row along x, a plane along x and y.
+int ensure_rows(mvd_session* s) {
+  auto& r = s->rc;
+  if (r.consts) return 0;
+  const Int3 n = s->img, q = r.plan->q;
+  const size_t row = sizeof(float2) * (size_t)r.plan->pitch;
+  const size_t nrows = (size_t)n.y * n.z, tile_elems = slab_elems(*r.plan, n.z) * r.tiles.size();
+  MVD_CHECK(r.rows.ensure(row * (nrows + 1)));
+  MVD_CHECK(r.planes.ensure(sizeof(float2) * (tile_elems + slab_elems(*r.plan, 1))));
+  float2* crow = r.rows.as<float2>() + (size_t)r.plan->pitch * nrows;
+  ConvGeom g{};
+  g.src = {1, 1, 1};
+  g.off = {0, 1, 1};  // outside the source: the constant everywhere
+  g.win = {r.win.x, 1, 1};
+  g.q = {q.x, 1, 1};
+  MVD_CHECK(launch_x_forward_any(*r.plan, g, s->d_psi.as<float>(), kGatherOne, crow, s->stream));
+  RowsPass y{};
+  y.kind = kPassYForward;
+  y.sp = r.plan;
+  y.n = n;
+  y.rows = r.rows.as<float2>();
+  y.planes = r.planes.as<float2>() + tile_elems;
+  y.off_y = n.y;
+  y.win_y = r.tiles[0].cnt + r.kd.y - 1;
+  y.nplanes = 1;
+  std::vector<PassLaunch> l;
+  LaunchTables tables;
+  int rc = build_rows_launches({y}, &tables, &l);
+  if (rc) return rc;
+  MVD_CHECK(tables.upload());
+  for (auto& L : l) MVD_CHECK(enqueue_pass_launch(L, s->stream));
+  MVD_CHECK(hipStreamSynchronize(s->stream));
+  r.consts = true;
+  return 0;
+}
+
+// The rows of the current estimate, on stream st.
+hipError_t rows_start(mvd_session* s, hipStream_t st) {
+  return launch_x_forward_any(*s->rc.plan, s->rc.geom, s->d_psi.as<float>(), kGatherMirror, s->rc.rows.as<float2>(),
+                              st);
 }
 
 // Launch lists of the block-batched iteration (one spectrum buffer per block).
@@ -957,6 +1261,24 @@ int build_block_batch(mvd_session* s) {
   auto& bb = s->bb;
   bb.view.clear();
   bb.ztab.clear();
+  bb.tables.host.clear();
+  if (s->rc.on) {
+    int rc = ensure_rows(s);
+    if (rc) return rc;
+    bb.view.resize(s->nviews);
+    for (int v = 0; v < s->nviews; ++v)
+      for (int conv = 0; conv < 2; ++conv) {
+        std::vector<RowsPass> pass[3];
+        std::vector<PassDesc> xinv;
+        rows_pass_descs(s, v, conv, pass, &xinv);
+        for (auto& p : pass)
+          if ((rc = build_rows_launches(p, &bb.tables, &bb.view[v]))) return rc;
+        if ((rc = build_pass_launches(xinv, &bb.tables, &bb.view[v]))) return rc;
+      }
+    MVD_CHECK(bb.tables.upload());
+    bb.built = bb.enabled = true;
+    return 0;
+  }
   size_t nb = 0, elems = 0;
   for (auto& v : s->views) {
     nb = std::max(nb, v.blocks.size());
@@ -1005,11 +1327,12 @@ int build_block_batch(mvd_session* s) {
         }
       }
       for (int p = 0; p < 5; ++p) {
-        int rc = build_pass_launches(pass[p], &bb.view[v], p == 0 && planned ? &tasks : nullptr,
+        int rc = build_pass_launches(pass[p], &bb.tables, &bb.view[v], p == 0 && planned ? &tasks : nullptr,
                                      sep && p < 2 ? &ptasks : nullptr, wide);
         if (rc) return rc;
       }
     }
+  MVD_CHECK(bb.tables.upload());
   return 0;
 }
 
@@ -1388,8 +1711,22 @@ int build_geometry(mvd_session* s, int v) {
 
 int view_spectra(mvd_session* s, int v) {
   mvd_session::View& view = s->views[v];
-  int rc = kernel_spectrum(s, *view.plan, view.k1, view.kd, &view.k1hat, &view.k1dc);
+  view.hat_ready = false;
+  int rc;
+  if (s->rc.on && !s->rc.shared) {
+    const ShapePlan& sp = *s->rc.plan;
+    const std::pair<const std::vector<float>*, DeviceBuf*> hats[2] = {{&view.k1, &view.r1hat}, {&view.k2, &view.r2hat}};
+    for (auto& h : hats) {
+      rc = kernel_spectrum(s, sp, *h.first, view.kd, &s->rc.plain);
+      if (rc) return rc;
+      MVD_CHECK(h.second->ensure(sizeof(float2) * slab_elems(sp, sp.q.z)));
+      MVD_CHECK(launch_to_slabs(sp, s->rc.plain.as<float2>(), h.second->as<float2>(), s->stream));
+    }
+    return 0;
+  }
+  rc = kernel_spectrum(s, *view.plan, view.k1, view.kd, &view.k1hat, &view.k1dc);
   if (rc) return rc;
+  view.hat_ready = true;
   return kernel_spectrum(s, *view.plan, view.k2, view.kd, &view.k2hat);
 }
 
@@ -1400,7 +1737,8 @@ int ensure_workspace(mvd_session* s) {
     spec = std::max<size_t>(spec, (size_t)view.plan->spectrum_elems());
     parts = std::max(parts, view.nwg_update);
   }
-  MVD_CHECK(s->d_spec.ensure(sizeof(float2) * spec));
+  if (s->rc.on) parts = std::max(parts, s->rc.nwg);
+  else MVD_CHECK(s->d_spec.ensure(sizeof(float2) * spec));
   MVD_CHECK(s->d_part_sum.ensure(sizeof(double) * parts));
   MVD_CHECK(s->d_part_max.ensure(sizeof(float) * parts));
   return 0;
@@ -1649,7 +1987,10 @@ int mvd_prepare(mvd_session* s, int psf_type, double lambda, const int* block_xy
   for (int v = 0; v < s->nviews; ++v) {
     int rc = build_geometry(s, v);
     if (rc) return rc;
-    rc = view_spectra(s, v);
+  }
+  if (int rc = plan_rows(s)) return rc;
+  for (int v = 0; v < s->nviews; ++v) {
+    int rc = view_spectra(s, v);
     if (rc) return rc;
   }
   int rc = ensure_workspace(s);
@@ -1674,7 +2015,7 @@ int mvd_set_psf(mvd_session* s, int view, const float* psf) {
   auto& v = s->views[view];
   v.psf_raw.assign(psf, psf + v.k1.size());
   v.k1 = v.psf_raw;
-  s->bb.built = false;
+  if (!s->rc.on) s->bb.built = false;  // (by rows: the launch lists name the same buffers)
   int rc = init_view(s, view);
   if (rc) return rc;
   return view_spectra(s, view);
@@ -1692,7 +2033,7 @@ int mvd_set_psfs(mvd_session* s, const float* const* psfs) {
     view.k1 = view.psf_raw;
     norm_img(view.k1, s->norm_threads);
   }
-  s->bb.built = false;
+  if (!s->rc.on) s->bb.built = false;
   for (int v = 0; v < s->nviews; ++v) {
     int rc = init_view(s, v, false);
     if (rc) return rc;
@@ -1759,6 +2100,11 @@ int mvd_iterate(mvd_session* s, int n, double* stats) {
     int rc = build_block_batch(s);
     if (rc) return rc;
   }
+  if (s->rc.on) {
+    s->timer.begin(s->stream);
+    MVD_CHECK(rows_start(s, s->stream));
+    s->timer.end(s->stream, kTXForward);
+  }
   // blocks of a view together: per pass one launch for all blocks
   for (int it = 0; s->bb.enabled && it < n; ++it) {
     for (int v = 0; v < s->nviews; ++v) {
@@ -1768,7 +2114,8 @@ int mvd_iterate(mvd_session* s, int n, double* stats) {
         s->timer.end(s->stream, L.timing);
       }
       s->timer.begin(s->stream);
-      MVD_CHECK(launch_reduce_stats(s->d_part_sum.as<double>(), s->d_part_max.as<float>(), s->views[v].nwg_update,
+      MVD_CHECK(launch_reduce_stats(s->d_part_sum.as<double>(), s->d_part_max.as<float>(),
+                                    s->rc.on ? s->rc.nwg : s->views[v].nwg_update,
                                     s->d_stats.as<double>() + 2 * ((size_t)it * s->nviews + v), s->stream));
       s->timer.end(s->stream, kTReduce);
     }
@@ -2005,7 +2352,12 @@ int mvd_nll_grad_device(mvd_session* s, const float* psi, const float* const* ps
     // the kernel spectrum: the prepared view's own when the PSF is its kernel1
     const float2* Kh = nullptr;
     double Kdc = 0.0;
-    if (s->prepared && view.plan == spp && view.k1hat.p && pk == view.k1) {
+    if (s->prepared && view.plan == spp && pk == view.k1) {
+      if (!view.hat_ready) {
+        int rc = kernel_spectrum(s, sp, view.k1, k, &view.k1hat, &view.k1dc);
+        if (rc) return rc;
+        view.hat_ready = true;
+      }
       Kh = view.k1hat.as<float2>();
       Kdc = view.k1dc;
     } else {
@@ -2279,6 +2631,7 @@ struct mvd_batch {
   std::vector<mvd_session*> stacks;
   std::vector<std::vector<DeviceBuf>> spec;  // [stack][block]
   std::vector<PassLaunch> launches;
+  LaunchTables tables;
   DeviceBuf stats_iter, stats_hist;
   std::vector<int> stats_off;  // per stack, in doubles
   int total_stats = 0;
@@ -2344,6 +2697,7 @@ int mvd_batch_prepare(mvd_batch* b, int use_graph) {
   b->exec = nullptr;
   b->graph = nullptr;
   b->launches.clear();
+  b->tables.host.clear();
   b->spec.clear();
   b->stats_off.clear();
   int maxv = 0, tot = 0;
@@ -2355,6 +2709,11 @@ int mvd_batch_prepare(mvd_batch* b, int use_graph) {
     size_t nb = 0;
     for (auto& v : s->views) nb = std::max(nb, v.blocks.size());
     b->spec.emplace_back();
+    if (s->rc.on) {
+      int rc = ensure_rows(s);
+      if (rc) return rc;
+      continue;
+    }
     for (size_t i = 0; i < nb; ++i) {
       b->spec.back().emplace_back();
       size_t elems = 0;
@@ -2370,15 +2729,22 @@ int mvd_batch_prepare(mvd_batch* b, int use_graph) {
   for (int v = 0; v < maxv; ++v) {
     for (int conv = 0; conv < 2; ++conv) {
       std::vector<PassDesc> pass[5];
+      std::vector<RowsPass> rows[3];
       for (size_t si = 0; si < b->stacks.size(); ++si) {
         mvd_session* s = b->stacks[si];
         if (v >= s->nviews) continue;
+        if (s->rc.on) {
+          rows_pass_descs(s, v, conv, rows, &pass[4]);
+          continue;
+        }
         std::vector<float2*> spec;
         for (auto& buf : b->spec[si]) spec.push_back(buf.as<float2>());
         conv_pass_descs(s, v, conv, spec, pass);
       }
       for (int p = 0; p < 5; ++p) {
-        int rc = build_pass_launches(pass[p], &b->launches);
+        if (p > 0 && p < 4)
+          if (int rc = build_rows_launches(rows[p - 1], &b->tables, &b->launches)) return rc;
+        int rc = build_pass_launches(pass[p], &b->tables, &b->launches);
         if (rc) return rc;
       }
     }
@@ -2389,6 +2755,7 @@ int mvd_batch_prepare(mvd_batch* b, int use_graph) {
       if (v >= s->nviews) continue;
       int n = 0;
       for (auto& g : s->views[v].blocks) n += conv_inverse_workgroups(*s->views[v].plan, g);
+      if (s->rc.on) n = s->rc.nwg;
       red.push_back({s->d_part_sum.as<double>(), s->d_part_max.as<float>(), n,
                      b->stats_iter.as<double>() + b->stats_off[si] + 2 * v});
     }
@@ -2396,10 +2763,11 @@ int mvd_batch_prepare(mvd_batch* b, int use_graph) {
     L.reduce = true;
     L.timing = kTReduce;
     L.nitems = (int)red.size();
-    MVD_CHECK(L.items.ensure(sizeof(ReduceItem) * red.size()));
-    MVD_CHECK(hipMemcpy(L.items.p, red.data(), sizeof(ReduceItem) * red.size(), hipMemcpyHostToDevice));
+    L.tab = &b->tables;
+    L.items_at = b->tables.add(red.data(), sizeof(ReduceItem) * red.size());
     b->launches.push_back(std::move(L));
   }
+  MVD_CHECK(b->tables.upload());
   b->use_graph = use_graph != 0;
   if (b->use_graph) {
     MVD_CHECK(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
@@ -2426,6 +2794,8 @@ int mvd_batch_iterate(mvd_batch* b, int n, double* stats) {
   if (n == 0) return 0;
   DeviceGuard guard(b->device);
   MVD_CHECK(b->stats_hist.ensure(sizeof(double) * (size_t)b->total_stats * n));
+  for (auto* s : b->stacks)
+    if (s->rc.on) MVD_CHECK(rows_start(s, b->stream));
   for (int it = 0; it < n; ++it) {
     if (b->use_graph) {
       MVD_CHECK(hipGraphLaunch(b->exec, b->stream));
