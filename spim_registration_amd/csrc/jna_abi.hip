@@ -249,16 +249,16 @@ constexpr int64_t kNaTwElems = 4 * kNaMaxLen;  // tw_x | tw_y | tw_z | unused (k
 constexpr int64_t kNaSpecElems = (int64_t)((kNaMaxLen / 2 + 1 + 15) / 16 * 16) * kNaMaxLen * kNaMaxLen;
 constexpr int64_t kNaElems = kNaTwElems + 2 * kNaSpecElems;
 
-// Twiddle tables handed over by value in the kernel arguments (3 KB), so that
-// filling them needs no host-to-device copy.
-struct NaTwiddles {
-  float2 t[3 * kNaMaxLen];
-};
-static_assert(sizeof(NaTwiddles) <= 3200, "kernel argument size");
-
-__global__ void k_na_twiddles(float2* dst, NaTwiddles tw) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < 3 * kNaMaxLen) dst[i] = tw.t[i];
+// Twiddle tables exp(-2 pi i m / n) of the three lengths, rounded from double.
+// On the GPU: a host table of 3 x 64 entries in long double was a quarter of a
+// 64^3 call (78 us; the call is bound by the host's nine launches).
+__global__ void k_na_twiddles(float2* dst, Int3 q) {
+  const int axis = blockIdx.x, m = threadIdx.x;
+  const int n = axis == 0 ? q.x : axis == 1 ? q.y : q.z;
+  if (m >= n) return;
+  double s, c;
+  sincospi(-2.0 * m / n, &s, &c);
+  dst[axis * kNaMaxLen + m] = make_float2((float)c, (float)s);
 }
 
 }  // namespace
@@ -431,14 +431,11 @@ int mvd_convolution3d_inplace_noalloc(float* im, const int* imDim, const float* 
   sp.tw_y = base + kNaMaxLen;
   sp.tw_z = base + 2 * kNaMaxLen;
   float2* spec = base + kNaTwElems;
-  float2* kspec = spec + kNaSpecElems;
+  // the kernel's spectrum follows the block's, so that one y pass takes both
+  float2* kspec = spec + sp.spectrum_elems();
   if (sp.spectrum_elems() > kNaSpecElems) return set_error("internal: no-allocation spectrum size"), -2;
-  NaTwiddles tw{};
-  fill_twiddles(tw.t, q.x);
-  fill_twiddles(tw.t + kNaMaxLen, q.y);
-  fill_twiddles(tw.t + 2 * kNaMaxLen, q.z);
   (void)hipGetLastError();
-  hipLaunchKernelGGL(k_na_twiddles, dim3((3 * kNaMaxLen + 255) / 256), dim3(256), 0, st, base, tw);
+  hipLaunchKernelGGL(k_na_twiddles, dim3(3), dim3(kNaMaxLen), 0, st, base, q);
   e = hipGetLastError();
   // kernel spectrum (wrapped kernel, scaled by 1 / (qx qy qz)), then the block
   ConvGeom kg{};
@@ -446,9 +443,6 @@ int mvd_convolution3d_inplace_noalloc(float* im, const int* imDim, const float* 
   kg.win = q;
   kg.q = q;
   if (e == hipSuccess) e = launch_x_forward(sp, kg, kernel, kGatherKernelWrap, kspec, st);
-  if (e == hipSuccess) e = launch_y(sp, kspec, 0, q.z, 0, q.y, -1.f, st);
-  const float scale = (float)(1.0L / ((long double)q.x * q.y * q.z));
-  if (e == hipSuccess) e = launch_z(sp, kspec, nullptr, scale, 0, q.z, st);
   ConvGeom g{};
   g.src = bd;
   g.win = bd;
@@ -458,7 +452,10 @@ int mvd_convolution3d_inplace_noalloc(float* im, const int* imDim, const float* 
   EpilogueArgs ep{};
   ep.mode = kEpiStore;
   ep.dst = im;
-  if (e == hipSuccess) e = launch_xy_forward_passes(sp, g, im, kGatherZero, spec, st);
+  if (e == hipSuccess) e = launch_x_forward(sp, g, im, kGatherZero, spec, st);
+  if (e == hipSuccess) e = launch_y(sp, spec, 0, 2 * q.z, 0, q.y, -1.f, st);
+  const float scale = (float)(1.0L / ((long double)q.x * q.y * q.z));
+  if (e == hipSuccess) e = launch_z(sp, kspec, nullptr, scale, 0, q.z, st);
   if (e == hipSuccess) e = launch_z(sp, spec, kspec, 1.f, 0, bd.z, st);
   if (e == hipSuccess) e = launch_yx_inverse_passes(sp, g, spec, ep, st, nullptr);
   if (e != hipSuccess) return set_error(std::string("no-allocation convolution: ") + hipGetErrorString(e)), -2;
