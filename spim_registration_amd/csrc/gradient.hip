@@ -231,6 +231,34 @@ hipError_t launch_sum_to(const float* a, int64_t n, double* part, int nparts, do
 // double sum.
 __global__ void k_set_dc(float2* spec, const double* v) { spec[0] = make_float2((float)*v, 0.f); }
 
+__global__ void k_set_dc_value(float2* spec, float v) { spec[0] = make_float2(v, 0.f); }
+
+hipError_t launch_set_dc_value(float2* spec, float v, hipStream_t stream) {
+  (void)hipGetLastError();
+  hipLaunchKernelGGL(k_set_dc_value, dim3(1), dim3(1), 0, stream, spec, v);
+  return hipGetLastError();
+}
+
+// out[v][i] = base[v][i] times factors[v (nv - 1) + w][i], w = 0 .. nv - 2, in
+// that order (the compound kernels' products, MVDeconFFT.java:249-258).
+__global__ __launch_bounds__(kGThreads) void k_compound_product(const float* base, const float* factors, int nv,
+                                                               int64_t n, float* out) {
+  const int64_t i = blockIdx.x * (int64_t)kGThreads + threadIdx.x;
+  const int v = blockIdx.y;
+  if (i >= n) return;
+  float t = base[v * n + i];
+  for (int w = 0; w < nv - 1; ++w) t = factors[((int64_t)v * (nv - 1) + w) * n + i] * t;
+  out[v * n + i] = t;
+}
+
+hipError_t launch_compound_product(const float* base, const float* factors, int nv, int64_t n, float* out,
+                                   hipStream_t stream) {
+  (void)hipGetLastError();
+  hipLaunchKernelGGL(k_compound_product, dim3((unsigned)((n + kGThreads - 1) / kGThreads), nv), dim3(kGThreads), 0,
+                     stream, base, factors, nv, n, out);
+  return hipGetLastError();
+}
+
 hipError_t launch_set_dc(float2* spec, const double* v, hipStream_t stream) {
   (void)hipGetLastError();
   hipLaunchKernelGGL(k_set_dc, dim3(1), dim3(1), 0, stream, spec, v);

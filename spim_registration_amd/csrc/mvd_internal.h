@@ -364,6 +364,7 @@ struct PassDesc {
   float dir, scale;
   int xy;  // x passes of a fused x-y item (no separate y pass)
   bool any = false;  // x passes: the two-radix kernels also where the length has its own
+  bool by_item = false;  // z pass: no lines launch (the bits of a convolution by itself)
   // z pass in the lines kernel only: input planes through a table of plane
   // indices into the arena of spectra (nullptr: plane z of spec)
   const unsigned short* ztab = nullptr;
@@ -483,6 +484,10 @@ hipError_t launch_window_sum_to(const float* img, Int3 n, Int3 lo, Int3 wd, doub
                                 hipStream_t stream);
 // spec[0] = (float) *v (the zero-frequency value of a spectrum).
 hipError_t launch_set_dc(float2* spec, const double* v, hipStream_t stream);
+hipError_t launch_set_dc_value(float2* spec, float v, hipStream_t stream);
+// out[v] = base[v] times factors[v (nv - 1) + w] for w = 0 .. nv - 2 in order, n values each.
+hipError_t launch_compound_product(const float* base, const float* factors, int nv, int64_t n, float* out,
+                                   hipStream_t stream);
 
 // Resampling of one view into the bounding box with its blending weight
 // (transform.hip).  inv: row-packed 3x4 inverse affine map (bounding-box

@@ -320,34 +320,27 @@ static std::vector<std::pair<int64_t, int64_t>> portions(int64_t n, int k) {
   return p;
 }
 
-// Pairwise summation of doubles in input order (binary counter).
+// Pairwise summation of doubles in input order: level i holds the sum of 2^i
+// values while bit i of the count is set.
 class PairSum {
  public:
   void add(double a) {
-    size_t i = 0;
-    double s = a;
-    while (i < full_.size() && full_[i]) {
-      full_[i] = false;
-      s += v_[i];
+    int i = 0;
+    for (uint64_t c = count_++; c & 1; c >>= 1, ++i) {
+      a += v_[i];
       v_[i] = 0.0;
-      ++i;
     }
-    if (i == full_.size()) {
-      full_.push_back(false);
-      v_.push_back(0.0);
-    }
-    full_[i] = true;
-    v_[i] = s;
+    v_[i] = a;
   }
   double sum() const {
     double s = 0;
-    for (double x : v_) s += x;
+    for (double x : v_) s += x;  // (the levels above the highest are zero)
     return s;
   }
 
  private:
-  std::vector<bool> full_;
-  std::vector<double> v_;
+  uint64_t count_ = 0;
+  double v_[64] = {};
 };
 
 // AdjustInput.normImg (deconv/AdjustInput.java:50-100): k /= S where S sums
@@ -730,6 +723,18 @@ struct mvd_session {
   DeviceBuf g_rsum;  // partials and the double sum of one block's residual
   DeviceBuf g_crop, g_gpsi;
   bool g_gpsi_ready = false;
+  DeviceBuf d_kern;  // a kernel on its way to its spectrum
+  // Compound kernels (init_views): the kernels and bases, the kernels'
+  // spectra, and per ordered pair of views a work spectrum and two kernel-sized
+  // arrays; the launch lists name these buffers and last as long as they do.
+  struct Compound {
+    bool built = false;
+    int type = -1;
+    Int3 kd{};
+    DeviceBuf kern, spec, work, a, b, out;
+    LaunchTables tables;
+    std::vector<PassLaunch> kernels, conv;
+  } cp;
   PlanCache plans;
   Timer timer;
   // The blocks of a view convolved together: one launch per pass and kernel
@@ -820,7 +825,7 @@ int build_pass_launches(const std::vector<PassDesc>& descs, LaunchTables* tab, s
   // spectra of 2^31 bytes or more take the per-item kernel)
   std::map<std::pair<const float2*, const ShapePlan*>, int> kshare;
   for (auto& d : descs)
-    if (d.kind == kPassZConv && d.kspec && pass_is_fast(d) && d.sp->spectrum_elems() * 8 < (int64_t(1) << 31))
+    if (d.kind == kPassZConv && d.kspec && !d.by_item && pass_is_fast(d) && d.sp->spectrum_elems() * 8 < (int64_t(1) << 31))
       ++kshare[{d.kspec, d.sp}];
   std::map<std::tuple<int, int, int, uintptr_t>, std::vector<const PassDesc*>> groups;
   for (auto& d : descs) {
@@ -842,8 +847,8 @@ int build_pass_launches(const std::vector<PassDesc>& descs, LaunchTables* tab, s
     // (the 384-point lines kernel exists with plane tables only: without them
     // it needs more than 256 VGPRs; those items take the batched z kernel)
     uintptr_t lines = 0;
-    if (path == 1 && d.kind == kPassZConv && d.kspec && kshare[{d.kspec, d.sp}] > 1 &&
-        (d.ztab != nullptr || d.sp->q.z != 384))
+    if (path == 1 && d.kind == kPassZConv && d.kspec && !d.by_item &&
+        kshare[{d.kspec, d.sp}] > 1 && (d.ztab != nullptr || d.sp->q.z != 384))
       lines = reinterpret_cast<uintptr_t>(d.kspec);
     groups[{path, cls, d.kind == kPassXInverse ? d.e.mode : 0, lines}].push_back(&d);
   }
@@ -1396,7 +1401,7 @@ int kernel_spectrum(mvd_session* s, const ShapePlan& sp, const std::vector<float
   // register x passes store the padding as zeros with every row.
   if (!fast_size(sp.q.x / 2) && !any_size(sp.px))
     MVD_CHECK(hipMemsetAsync(out->p, 0, sizeof(float2) * sp.spectrum_elems(), s->stream));
-  DeviceBuf dk;
+  DeviceBuf& dk = s->d_kern;
   MVD_CHECK(dk.ensure(sizeof(float) * k.size()));
   MVD_CHECK(hipMemcpyAsync(dk.p, k.data(), sizeof(float) * k.size(), hipMemcpyHostToDevice, s->stream));
   ConvGeom g{};
@@ -1423,10 +1428,8 @@ int kernel_spectrum(mvd_session* s, const ShapePlan& sp, const std::vector<float
   // strongly than to the PSF values themselves near a fitted estimate.
   long double sum = 0.0L;
   for (float v : k) sum += v;
-  const float2 dc = make_float2((float)(sum / n), 0.f);
   if (dc_out) *dc_out = (double)(sum / n);
-  MVD_CHECK(hipMemcpyAsync(out->p, &dc, sizeof(dc), hipMemcpyHostToDevice, s->stream));
-  MVD_CHECK(hipStreamSynchronize(s->stream));
+  MVD_CHECK(launch_set_dc_value(out->as<float2>(), (float)(sum / n), s->stream));
   return 0;
 }
 
@@ -1507,6 +1510,170 @@ int init_view(mvd_session* s, int v, bool normalise = true) {
     }
     norm_img(e, s->norm_threads);
     view.k2 = inverted(e, view.kd);
+  }
+  return 0;
+}
+
+// MVDeconFFT.init of all views at once, k1 holding the kernels as given: view v
+// is prepared from its own normalised kernel1, the normalised ones of the views
+// before it, and of the views after it the ones as given (normalise_first
+// false, as the views are initialised one after another) or normalised too.
+//
+// The compound convolutions of all ordered pairs of views run in one launch per
+// pass and stay on the device; the products come back in one copy.  One
+// convolution at a time, 24 for four views, each has its allocations, copies and
+// waits: two refinement steps of four 200x180x120 views with 25x25x31 kernels took
+// 17.1 ms, most of it that; with all of them together 8.7 ms.
+// Kernels of several sizes, spectra of more than 512 MiB together, and buffers
+// that the device has no memory for are prepared view by view.
+int init_views(mvd_session* s, bool normalise_first) {
+  auto& V = s->views;
+  const int nv = s->nviews;
+  const Int3 kd = V[0].kd;
+  const bool eff = s->psf_type == MVD_PSF_EFFICIENT_BAYESIAN;
+  bool together = nv > 1 && (eff || s->psf_type == MVD_PSF_OPTIMIZATION_I);
+  for (auto& v : V) together = together && v.kd.x == kd.x && v.kd.y == kd.y && v.kd.z == kd.z;
+  ConvGeom g{};
+  g.src = g.eff_size = g.dst = kd;
+  g.off = {-kd.x / 2, -kd.y / 2, -kd.z / 2};
+  g.win = {2 * kd.x - 1, 2 * kd.y - 1, 2 * kd.z - 1};
+  g.q = fft_shape_for(g.win);
+  g.eff_local = {kd.x / 2, kd.y / 2, kd.z / 2};
+  const ShapePlan* sp = together ? s->plans.get(g.q) : nullptr;
+  // device order: the bases, then per set (the kernels of the views before, and
+  // of the views after) and view the kernel (eff) and its mirror image
+  const int per = eff ? 2 : 1, nspec = 2 * nv * per;
+  const size_t pairs = (size_t)nv * (nv - 1);
+  const int64_t kn = (int64_t)kd.x * kd.y * kd.z, elems = sp ? sp->spectrum_elems() : 0;
+  auto& c = s->cp;
+  const bool build = !c.built || c.type != s->psf_type || c.kd.x != kd.x || c.kd.y != kd.y || c.kd.z != kd.z;
+  together = sp && (pairs + nspec) * elems * sizeof(float2) <= (size_t(512) << 20) &&
+             (int64_t)nspec * g.q.z <= 65535;  // (one y pass over the planes of all kernels)
+  if (together && build) {
+    c.built = false;
+    const std::pair<DeviceBuf*, size_t> sizes[] = {{&c.kern, sizeof(float) * kn * (nv + nspec)},
+                                                   {&c.spec, sizeof(float2) * elems * nspec},
+                                                   {&c.work, sizeof(float2) * elems * pairs},
+                                                   {&c.a, sizeof(float) * kn * pairs},
+                                                   {&c.b, sizeof(float) * kn * pairs},
+                                                   {&c.out, sizeof(float) * kn * nv}};
+    for (auto& b : sizes) together = together && b.first->ensure(b.second) == hipSuccess;
+    if (!together) {
+      (void)hipGetLastError();
+      for (auto& b : sizes) *b.first = DeviceBuf();
+    }
+  }
+  if (!together) {
+    if (normalise_first)
+      for (auto& v : V) norm_img(v.k1, s->norm_threads);
+    for (int v = 0; v < nv; ++v) {
+      int rc = init_view(s, v, !normalise_first);
+      if (rc) return rc;
+    }
+    return 0;
+  }
+  std::vector<float> host((size_t)kn * (nv + nspec));
+  auto slot = [&](int set, int w, int inverse) { return nv + (set * nv + w) * per + (eff ? inverse : 0); };
+  auto put = [&](int at, const std::vector<float>& k) { std::copy(k.begin(), k.end(), host.begin() + at * kn); };
+  for (int w = 0; w < nv; ++w) {
+    const std::vector<float> given = V[w].k1;
+    norm_img(V[w].k1, s->norm_threads);
+    const std::vector<float> inv = inverted(V[w].k1, kd);
+    put(w, eff ? inv : V[w].k1);
+    for (int set = 0; set < 2; ++set) {
+      const bool raw = set == 1 && !normalise_first;
+      if (eff) put(slot(set, w, 0), raw ? given : V[w].k1);
+      put(slot(set, w, 1), raw ? inverted(given, kd) : inv);
+    }
+  }
+  hipStream_t st = s->stream;
+  if (build) {
+    // finite row padding where the x pass leaves it unwritten
+    MVD_CHECK(hipMemsetAsync(c.spec.p, 0, sizeof(float2) * elems * nspec, st));
+    MVD_CHECK(hipMemsetAsync(c.work.p, 0, sizeof(float2) * elems * pairs, st));
+    c.tables.host.clear();
+    c.kernels.clear();
+    c.conv.clear();
+    std::vector<PassDesc> xk;
+    for (int i = 0; i < nspec; ++i) {
+      PassDesc d{};
+      d.kind = kPassXForward;
+      d.sp = sp;
+      d.g.src = kd;
+      d.g.win = d.g.q = g.q;
+      d.gather = kGatherKernelWrap;
+      d.src = c.kern.as<float>() + (nv + i) * kn;
+      d.spec = c.spec.as<float2>() + i * elems;
+      xk.push_back(d);
+    }
+    int rc = build_pass_launches(xk, &c.tables, &c.kernels);
+    if (rc) return rc;
+    for (int step = 0; step < per; ++step) {
+      std::vector<PassDesc> pass[5];
+      int p = 0;
+      for (int v = 0; v < nv; ++v)
+        for (int w = 0; w < nv; ++w) {
+          if (w == v) continue;
+          PassDesc d{};
+          d.sp = sp;
+          d.g = g;
+          d.spec = c.work.as<float2>() + p * elems;
+          d.kspec = c.spec.as<float2>() + (slot(w < v ? 0 : 1, w, eff ? step : 1) - nv) * elems;
+          d.src = step == 0 ? c.kern.as<float>() + v * kn : c.a.as<float>() + p * kn;
+          d.gather = kGatherZero;
+          d.scale = 1.f;
+          d.kind = kPassXForward;
+          pass[0].push_back(d);
+          d.kind = kPassYForward;
+          d.zhi = g.q.z;
+          d.yhi = g.q.y;
+          d.dir = -1.f;
+          pass[1].push_back(d);
+          d.kind = kPassZConv;
+          d.by_item = true;
+          d.zlo = g.eff_local.z;
+          d.zhi = d.zlo + kd.z;
+          pass[2].push_back(d);
+          d.kind = kPassYInverse;
+          d.ylo = g.eff_local.y;
+          d.yhi = d.ylo + kd.y;
+          d.dir = 1.f;
+          pass[3].push_back(d);
+          d.kind = kPassXInverse;
+          d.e.mode = kEpiStore;
+          d.e.dst = (step + 1 == per ? c.b : c.a).as<float>() + p * kn;
+          pass[4].push_back(d);
+          ++p;
+        }
+      for (auto& ds : pass)
+        if ((rc = build_pass_launches(ds, &c.tables, &c.conv))) return rc;
+    }
+    MVD_CHECK(c.tables.upload());
+    c.type = s->psf_type;
+    c.kd = kd;
+    c.built = true;
+  }
+  MVD_CHECK(hipMemcpyAsync(c.kern.p, host.data(), sizeof(float) * host.size(), hipMemcpyHostToDevice, st));
+  for (auto& L : c.kernels) MVD_CHECK(enqueue_pass_launch(L, st));
+  // the spectra lie one after another: one y pass over the planes of all
+  MVD_CHECK(launch_y(*sp, c.spec.as<float2>(), 0, nspec * g.q.z, 0, g.q.y, -1.f, st));
+  const long double n = (long double)g.q.x * g.q.y * g.q.z;
+  for (int i = 0; i < nspec; ++i) {
+    float2* spec = c.spec.as<float2>() + i * elems;
+    MVD_CHECK(launch_z(*sp, spec, nullptr, (float)(1.0L / n), 0, g.q.z, st));
+    long double sum = 0.0L;  // the exact zero frequency (kernel_spectrum)
+    for (int64_t j = 0; j < kn; ++j) sum += host[(nv + i) * kn + j];
+    MVD_CHECK(launch_set_dc_value(spec, (float)(sum / n), st));
+  }
+  for (auto& L : c.conv) MVD_CHECK(enqueue_pass_launch(L, st));
+  MVD_CHECK(launch_compound_product(c.kern.as<float>(), c.b.as<float>(), nv, kn, c.out.as<float>(), st));
+  std::vector<float> prod((size_t)kn * nv);
+  MVD_CHECK(hipMemcpyAsync(prod.data(), c.out.p, sizeof(float) * prod.size(), hipMemcpyDeviceToHost, st));
+  MVD_CHECK(hipStreamSynchronize(st));
+  for (int v = 0; v < nv; ++v) {
+    std::vector<float> t(prod.begin() + v * kn, prod.begin() + (v + 1) * kn);
+    norm_img(t, s->norm_threads);
+    V[v].k2 = eff ? t : inverted(t, kd);
   }
   return 0;
 }
@@ -1980,10 +2147,7 @@ int mvd_prepare(mvd_session* s, int psf_type, double lambda, const int* block_xy
   }
   for (auto& v : s->views) v.k1 = v.psf_raw;
   // MVDeconInput.init: views in order
-  for (int v = 0; v < s->nviews; ++v) {
-    int rc = init_view(s, v);
-    if (rc) return rc;
-  }
+  if (int rc = init_views(s, false)) return rc;
   for (int v = 0; v < s->nviews; ++v) {
     int rc = build_geometry(s, v);
     if (rc) return rc;
@@ -1995,6 +2159,7 @@ int mvd_prepare(mvd_session* s, int psf_type, double lambda, const int* block_xy
   }
   int rc = ensure_workspace(s);
   if (rc) return rc;
+  MVD_CHECK(hipStreamSynchronize(s->stream));
   s->prepared = true;
   return 0;
 }
@@ -2018,7 +2183,9 @@ int mvd_set_psf(mvd_session* s, int view, const float* psf) {
   if (!s->rc.on) s->bb.built = false;  // (by rows: the launch lists name the same buffers)
   int rc = init_view(s, view);
   if (rc) return rc;
-  return view_spectra(s, view);
+  if ((rc = view_spectra(s, view))) return rc;
+  MVD_CHECK(hipStreamSynchronize(s->stream));
+  return 0;
 }
 
 int mvd_set_psfs(mvd_session* s, const float* const* psfs) {
@@ -2031,15 +2198,14 @@ int mvd_set_psfs(mvd_session* s, const float* const* psfs) {
     auto& view = s->views[v];
     view.psf_raw.assign(psfs[v], psfs[v] + view.k1.size());
     view.k1 = view.psf_raw;
-    norm_img(view.k1, s->norm_threads);
   }
   if (!s->rc.on) s->bb.built = false;
+  if (int rc = init_views(s, true)) return rc;
   for (int v = 0; v < s->nviews; ++v) {
-    int rc = init_view(s, v, false);
-    if (rc) return rc;
-    rc = view_spectra(s, v);
+    int rc = view_spectra(s, v);
     if (rc) return rc;
   }
+  MVD_CHECK(hipStreamSynchronize(s->stream));
   return 0;
 }
 
