@@ -497,6 +497,7 @@ constexpr int kBlendLutSize = 1001;
 struct TransformArgs {
   const float* raw;
   int rsize[3];
+  float rlim[3];  // set by launch_transform_view
   double inv[12];
   float off[3];
   int nx, ny, nz;

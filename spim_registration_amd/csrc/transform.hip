@@ -3,8 +3,8 @@
 // (deconv/TransformInputAndWeights.java:100-135, deconv/TransformInput.java:69-95,
 //  spim/process/fusion/weights/BlendingRealRandomAccess.java:44-121).
 //
-// Threads run along x (the image and weight stores of a wavefront are 256
-// contiguous bytes each), four output rows per thread.  The arithmetic
+// A wavefront takes 64 voxels along x or a tile of 16 x 4 (whichever reads fewer
+// raw lines), four output rows per thread.  The arithmetic
 // keeps the reference's types and order so that results are bit-identical to
 // the CPU restatement: the inverse affine map in double, evaluated left to
 // right without fused multiply-adds and rounded to float; trilinear weights in
@@ -13,6 +13,7 @@
 // table in double.  The inputs are read through the texture-less vector path:
 // the eight corners of neighbouring voxels overlap, so they hit L1/L2 and the
 // HBM traffic is about one read of the raw view plus the two outputs.
+#include <algorithm>
 #include <cmath>
 #include <mutex>
 #include <string>
@@ -64,55 +65,80 @@ __device__ __forceinline__ float blend_weight(const float t[3], const int size[3
   return m;
 }
 
+// Two neighbouring values of a raw row, at any multiple of four bytes.
+struct __attribute__((packed, aligned(4))) RawPair {
+  float a, b;
+};
+
 // Trilinear interpolation over the mirror-single extension, for 0 <= t < size
 // (the caller checks): the lower corner is in range and the upper one only
 // leaves it at the far face, where the mirror maps n to n - 2 (n = 1: 0).
+// The two corners of a row are one 8-byte load; at the far face it starts one
+// voxel lower and its values change places (the mirror of n is n - 2).  The
+// integer and fractional parts are taken in float: t >= 0, so both are exact.
 // kOff32: the raw view spans fewer than 2^32 bytes, so corner addresses are
 // 32-bit byte offsets from the (uniform) base.
+struct Corners {
+  RawPair q00, q10, q01, q11;  // rows (y0, z0), (y1, z0), (y0, z1), (y1, z1)
+  bool far;                    // pairs that start one voxel lower
+};
+
 template <bool kOff32>
-__device__ __forceinline__ float trilinear(const float* __restrict__ raw, const int size[3], const float t[3]) {
+__device__ __forceinline__ Corners gather(const float* __restrict__ raw, const int size[3], const float t[3]) {
+  Corners c;
+  const int x0 = (int)t[0], y0 = (int)t[1], z0 = (int)t[2];
+  const int y1 = y0 + 1 < size[1] ? y0 + 1 : (size[1] > 1 ? size[1] - 2 : 0);
+  const int z1 = z0 + 1 < size[2] ? z0 + 1 : (size[2] > 1 ? size[2] - 2 : 0);
+  const bool pairs = size[0] > 1;
+  c.far = pairs && x0 + 1 == size[0];
+  const int xb = c.far ? x0 - 1 : x0;
+  if constexpr (kOff32) {
+    const uint32_t sx = (uint32_t)size[0], sxy = (uint32_t)size[0] * (uint32_t)size[1];
+    const uint32_t at = (uint32_t)xb * 4u;
+    const uint32_t r00 = (y0 * sx + z0 * sxy) * 4u + at, r10 = (y1 * sx + z0 * sxy) * 4u + at;
+    const uint32_t r01 = (y0 * sx + z1 * sxy) * 4u + at, r11 = (y1 * sx + z1 * sxy) * 4u + at;
+    if (pairs) {
+      c.q00 = *gbyte((const RawPair*)raw, r00);
+      c.q10 = *gbyte((const RawPair*)raw, r10);
+      c.q01 = *gbyte((const RawPair*)raw, r01);
+      c.q11 = *gbyte((const RawPair*)raw, r11);
+    } else {
+      c.q00.a = c.q00.b = *gbyte(raw, r00);
+      c.q10.a = c.q10.b = *gbyte(raw, r10);
+      c.q01.a = c.q01.b = *gbyte(raw, r01);
+      c.q11.a = c.q11.b = *gbyte(raw, r11);
+    }
+  } else {
+    const int64_t sx = size[0], sxy = (int64_t)size[0] * size[1];
+    const auto g = gmem(raw) + xb;
+    const int64_t r00 = y0 * sx + z0 * sxy, r10 = y1 * sx + z0 * sxy;
+    const int64_t r01 = y0 * sx + z1 * sxy, r11 = y1 * sx + z1 * sxy;
+    const int n = pairs ? 1 : 0;
+    c.q00 = {g[r00], g[r00 + n]};
+    c.q10 = {g[r10], g[r10 + n]};
+    c.q01 = {g[r01], g[r01 + n]};
+    c.q11 = {g[r11], g[r11 + n]};
+  }
+  return c;
+}
+
+__device__ __forceinline__ float trilinear(Corners c, const float t[3]) {
 #pragma clang fp contract(off)
-  const double p0 = t[0], p1 = t[1], p2 = t[2];
-  const double f0 = floor(p0), f1 = floor(p1), f2 = floor(p2);
-  const double w0 = p0 - f0, w0i = 1.0 - w0;
-  const double w1 = p1 - f1, w1i = 1.0 - w1;
-  const double w2 = p2 - f2, w2i = 1.0 - w2;
+  const double w0 = (double)(t[0] - floorf(t[0])), w0i = 1.0 - w0;
+  const double w1 = (double)(t[1] - floorf(t[1])), w1i = 1.0 - w1;
+  const double w2 = (double)(t[2] - floorf(t[2])), w2i = 1.0 - w2;
   // NLinearInterpolator3D weights: products in the order x, y, z
   const double a00 = w0i * w1i, a10 = w0 * w1i, a01 = w0i * w1, a11 = w0 * w1;
   const double w000 = a00 * w2i, w100 = a10 * w2i, w010 = a01 * w2i, w110 = a11 * w2i;
   const double w001 = a00 * w2, w101 = a10 * w2, w011 = a01 * w2, w111 = a11 * w2;
-  const int x0 = (int)f0, y0 = (int)f1, z0 = (int)f2;
-  const int x1 = x0 + 1 < size[0] ? x0 + 1 : (size[0] > 1 ? size[0] - 2 : 0);
-  const int y1 = y0 + 1 < size[1] ? y0 + 1 : (size[1] > 1 ? size[1] - 2 : 0);
-  const int z1 = z0 + 1 < size[2] ? z0 + 1 : (size[2] > 1 ? size[2] - 2 : 0);
-  float v000, v100, v110, v010, v011, v111, v101, v001;
-  if constexpr (kOff32) {
-    const uint32_t sx = (uint32_t)size[0], sxy = (uint32_t)size[0] * (uint32_t)size[1];
-    const uint32_t r00 = (y0 * sx + z0 * sxy) * 4u, r10 = (y1 * sx + z0 * sxy) * 4u;
-    const uint32_t r01 = (y0 * sx + z1 * sxy) * 4u, r11 = (y1 * sx + z1 * sxy) * 4u;
-    const uint32_t c0 = (uint32_t)x0 * 4u, c1 = (uint32_t)x1 * 4u;
-    v000 = *gbyte(raw, r00 + c0);
-    v100 = *gbyte(raw, r00 + c1);
-    v110 = *gbyte(raw, r10 + c1);
-    v010 = *gbyte(raw, r10 + c0);
-    v011 = *gbyte(raw, r11 + c0);
-    v111 = *gbyte(raw, r11 + c1);
-    v101 = *gbyte(raw, r01 + c1);
-    v001 = *gbyte(raw, r01 + c0);
-  } else {
-    const int64_t sx = size[0], sxy = (int64_t)size[0] * size[1];
-    const int64_t r00 = y0 * sx + z0 * sxy, r10 = y1 * sx + z0 * sxy;
-    const int64_t r01 = y0 * sx + z1 * sxy, r11 = y1 * sx + z1 * sxy;
-    const auto g = gmem(raw);
-    v000 = g[r00 + x0];
-    v100 = g[r00 + x1];
-    v110 = g[r10 + x1];
-    v010 = g[r10 + x0];
-    v011 = g[r11 + x0];
-    v111 = g[r11 + x1];
-    v101 = g[r01 + x1];
-    v001 = g[r01 + x0];
+  if (c.far) {
+    c.q00 = {c.q00.b, c.q00.a};
+    c.q10 = {c.q10.b, c.q10.a};
+    c.q01 = {c.q01.b, c.q01.a};
+    c.q11 = {c.q11.b, c.q11.a};
   }
+  const float v000 = c.q00.a, v100 = c.q00.b, v010 = c.q10.a, v110 = c.q10.b;
+  const float v001 = c.q01.a, v101 = c.q01.b, v011 = c.q11.a, v111 = c.q11.b;
   // FloatType accumulation in the interpolator's corner order
   float acc = (float)((double)v000 * w000);
   acc = acc + (float)((double)v100 * w100);
@@ -125,19 +151,29 @@ __device__ __forceinline__ float trilinear(const float* __restrict__ raw, const 
   return acc;
 }
 
-// A workgroup covers kTfThreads consecutive x of kTfVox consecutive output rows
-// (same z); each thread walks its column down the rows, so the raw rows that
-// two neighbouring output rows share are fetched once into this CU's cache
-// (every store instruction of a wavefront still writes 256 contiguous bytes).
+// A wavefront covers LX x LY x LZ output voxels, a workgroup four of them along
+// x, each thread kTfVox of them LY rows apart (same z), so the raw rows that
+// neighbouring output rows share are fetched once into this CU's cache.
+//
+// A gather costs the cache one cycle per raw line that the wavefront's 64 voxels
+// touch: 64 voxels along x of a view turned by 60 degrees lie in about 30 raw
+// rows, 16 x 4 of them in 11.  512x512x256 with weights from 512x512x128 at 60
+// degrees: 535 us with 64 voxels along x and eight 4-byte loads each (the L1 busy
+// 93 % of the time), 435 us now.  What is left is arithmetic, 70 FP64 instructions
+// a voxel; two or four rows in flight per thread (70 VGPRs) measured 430 to 445,
+// eight or sixteen rows per thread 450 to 466.
 constexpr int kTfVox = 4;
 
-template <bool kOff32>
+template <bool kOff32, int LX, int LY, int LZ>
 __global__ __launch_bounds__(kTfThreads) void k_transform_view(TransformArgs a, int chunks, int ygroups) {
 #pragma clang fp contract(off)
-  const int zy = blockIdx.x / chunks;  // z * ygroups + y group
-  const int x = (blockIdx.x - zy * chunks) * kTfThreads + threadIdx.x;
-  if (x >= a.nx) return;
-  const int z = zy / ygroups, y0 = (zy - z * ygroups) * kTfVox;
+  static_assert(LX * LY * LZ == 64, "one wavefront");
+  const int zy = blockIdx.x / chunks;  // z group * ygroups + y group
+  const int lane = threadIdx.x % 64, wave = threadIdx.x / 64;
+  const int x = ((blockIdx.x - zy * chunks) * 4 + wave) * LX + lane % LX;
+  const int zg = zy / ygroups, y0 = (zy - zg * ygroups) * (kTfVox * LY) + lane / LX % LY;
+  const int z = zg * LZ + lane / (LX * LY);
+  if (x >= a.nx || z >= a.nz) return;
   // cursor position (float) + offset (int): TransformInput.java:79-83;
   // AffineTransform3D.applyInverse: (float)(m0*s0 + m1*s1 + m2*s2 + m3), left
   // to right in double -- m0*s0 and m2*s2 are the column's terms
@@ -150,24 +186,27 @@ __global__ __launch_bounds__(kTfThreads) void k_transform_view(TransformArgs a, 
   }
 #pragma unroll 1
   for (int k = 0; k < kTfVox; ++k) {
-    const int y = y0 + k;
+    const int y = y0 + k * LY;
     if (y >= a.ny) break;
     const double s1 = (double)((float)y + a.off[1]);
     float t[3];
 #pragma unroll
     for (int r = 0; r < 3; ++r) t[r] = (float)(((ra[r] + a.inv[4 * r + 1] * s1) + rc[r]) + a.inv[4 * r + 3]);
     const int64_t o = ((int64_t)z * a.ny + y) * a.nx + x;
+    // FusionHelper.intersects
+    const bool in = a.out_img && t[0] >= 0.f && t[1] >= 0.f && t[2] >= 0.f && t[0] < a.rlim[0] && t[1] < a.rlim[1] &&
+                    t[2] < a.rlim[2];
+    Corners c;
+    if (in) c = gather<kOff32>(a.raw, a.rsize, t);  // in flight under the weight's arithmetic
+    if (a.out_w) gmem(a.out_w)[o] = blend_weight(t, a.rsize, a.border, a.range, a.lut);
     if (a.out_img) {
       float v = 0.f;  // outside the view: the reference's new image keeps 0
-      // FusionHelper.intersects
-      if (t[0] >= 0.f && t[1] >= 0.f && t[2] >= 0.f && (double)t[0] < (double)a.rsize[0] &&
-          (double)t[1] < (double)a.rsize[1] && (double)t[2] < (double)a.rsize[2]) {
-        const float r = trilinear<kOff32>(a.raw, a.rsize, t);
+      if (in) {
+        const float r = trilinear(c, t);
         v = r != r ? r : (r > kMinValueF ? r : kMinValueF);  // Math.max(minValue, r)
       }
       gmem(a.out_img)[o] = v;
     }
-    if (a.out_w) gmem(a.out_w)[o] = blend_weight(t, a.rsize, a.border, a.range, a.lut);
   }
 }
 
@@ -207,18 +246,74 @@ const char* check_transform_args(const TransformArgs& a) {
   return nullptr;
 }
 
-hipError_t launch_transform_view(const TransformArgs& a, hipStream_t stream) {
-  const int chunks = (a.nx + kTfThreads - 1) / kTfThreads;
-  const int ygroups = (a.ny + kTfVox - 1) / kTfVox;
-  const int64_t wgs = (int64_t)ygroups * a.nz * chunks;
-  const bool off32 = (int64_t)a.rsize[0] * a.rsize[1] * a.rsize[2] * 4 < (int64_t(1) << 32);
-  (void)hipGetLastError();
-  if (off32)
-    hipLaunchKernelGGL(k_transform_view<true>, dim3((unsigned)wgs), dim3(kTfThreads), 0, stream, a, chunks,
-                       ygroups);
+namespace {
+
+template <int LX, int LY, int LZ>
+int64_t tile_wgs(const TransformArgs& a, int* chunks, int* ygroups) {
+  *chunks = (a.nx + 4 * LX - 1) / (4 * LX);
+  *ygroups = (a.ny + kTfVox * LY - 1) / (kTfVox * LY);
+  return (int64_t)*chunks * *ygroups * ((a.nz + LZ - 1) / LZ);
+}
+
+// Lines that the wavefront's loads (four of raw pairs) and store touch: a row of
+// voxels along x enters a new raw row with every step in the raw y and z, and
+// the tile as a whole cannot touch more than its bounding box holds.
+template <int LX, int LY, int LZ>
+double tile_lines(const TransformArgs& a) {
+  auto m = [&](int r, int c) { return std::fabs(a.inv[4 * r + c]); };
+  double box = 1, path = 1;
+  for (int r = 0; r < 3; ++r) {
+    const double per_line = r == 0 ? 32.0 : 1.0;
+    box *= 1 + ((LX - 1) * m(r, 0) + (LY - 1) * m(r, 1) + (LZ - 1) * m(r, 2)) / per_line;
+    path += (LX - 1) * m(r, 0) / per_line;
+  }
+  return 4 * std::min({64.0, box, LY * LZ * path}) + LY * LZ * std::max(1.0, LX / 32.0);
+}
+
+template <int LX, int LY, int LZ>
+void launch_tile(const TransformArgs& a, hipStream_t stream) {
+  int chunks, ygroups;
+  const int64_t wgs = tile_wgs<LX, LY, LZ>(a, &chunks, &ygroups);
+  if ((int64_t)a.rsize[0] * a.rsize[1] * a.rsize[2] * 4 < (int64_t(1) << 32))
+    hipLaunchKernelGGL((k_transform_view<true, LX, LY, LZ>), dim3((unsigned)wgs), dim3(kTfThreads), 0, stream, a,
+                       chunks, ygroups);
   else
-    hipLaunchKernelGGL(k_transform_view<false>, dim3((unsigned)wgs), dim3(kTfThreads), 0, stream, a, chunks,
-                       ygroups);
+    hipLaunchKernelGGL((k_transform_view<false, LX, LY, LZ>), dim3((unsigned)wgs), dim3(kTfThreads), 0, stream, a,
+                       chunks, ygroups);
+}
+
+}  // namespace
+
+hipError_t launch_transform_view(const TransformArgs& args, hipStream_t stream) {
+  TransformArgs a = args;
+  for (int d = 0; d < 3; ++d) {  // the smallest float >= size: t < size for a float t
+    a.rlim[d] = (float)a.rsize[d];
+    if ((double)a.rlim[d] < (double)a.rsize[d]) a.rlim[d] = std::nextafterf(a.rlim[d], INFINITY);
+  }
+  // The tile of fewest lines, counting the work of lanes outside the output.
+  // Rows also without an image (nothing is gathered), and where a step in x hardly
+  // moves along the raw x: there the tile's planes, a power of two apart in many
+  // views, compete for the same cache sets.  512x512x256 from 512x512x128, turned
+  // about y, rows against 16 x 4: 0 degrees 375 and 390 us, 20 401 and 400, 60 456
+  // and 435, 70 457 and 450, 80 455 and 468, 90 427 and 558; 500x490x250 from
+  // 500x490x125: 20 439 and 375, 45 526 and 416, 60 500 and 433, 90 443 and 434.
+  int c, g;
+  const double rows = (double)tile_wgs<64, 1, 1>(a, &c, &g);
+  double best = tile_lines<64, 1, 1>(a) * rows;
+  int tile = 0;
+  if (a.out_img && std::fabs(a.inv[0]) >= 0.2) {
+    if (const double n = (double)tile_wgs<16, 1, 4>(a, &c, &g); n < 2147483648.0 && tile_lines<16, 1, 4>(a) * n < best)
+      best = tile_lines<16, 1, 4>(a) * n, tile = 1;
+    if (const double n = (double)tile_wgs<16, 4, 1>(a, &c, &g); n < 2147483648.0 && tile_lines<16, 4, 1>(a) * n < best)
+      tile = 2;
+  }
+  (void)hipGetLastError();
+  if (tile == 1)
+    launch_tile<16, 1, 4>(a, stream);
+  else if (tile == 2)
+    launch_tile<16, 4, 1>(a, stream);
+  else
+    launch_tile<64, 1, 1>(a, stream);
   return hipGetLastError();
 }
 
