@@ -314,6 +314,7 @@ __device__ __forceinline__ void x_any_inverse_body(const XAnyInvParams& P, int b
         float w = in1[u];
         if (e.weight_mode == kWeightVirtual) w = (float)java_min(1.0, (double)w / (double)in2[u] * e.osem);
         const float next = rl_next_value(in0[u], val, w, e.lambda, inv_lambda);
+        if (e.keep) gmem(e.keep)[base[u]] = in0[u];
         *dst = next;
         if (r_rows) fbuf[vofs[u]] = next;
         const float change = fabsf(next - in0[u]);
@@ -367,6 +368,26 @@ __device__ __forceinline__ void x_any_inverse_body(const XAnyInvParams& P, int b
     // the x transform of the window rows
     const int l = (int)__umulhi((unsigned)threadIdx.x, f.mb), j = threadIdx.x - l * f.b;
     __syncthreads();
+    if ((EPI == kEpiQuotient || EPI == kEpiUpdate) && e.part_sq) {
+      // the rows' energies, a wave per piece, from LDS once more (6 views of
+      // 512x512x256: quotient 249 -> 266 us, update 418 -> 431)
+      const int pieces = energy_pieces(nx);
+      for (int p = wave; p < pieces; p += nw) {
+        const int x = p * kEnergyPiece + lane;
+        const float* q = fbuf + g.eff_local.x + (x < nx ? x : 0);
+        float s = 0.f;
+        for (int r = 0; r < live_rows; r += 4) {
+          float v[4];
+#pragma unroll
+          for (int u = 0; u < 4; ++u) v[u] = q[2 * min(r + u, live_rows - 1) * P.slots];
+#pragma unroll
+          for (int u = 0; u < 4; ++u) s += r + u < live_rows ? v[u] * v[u] : 0.f;
+        }
+        if (x >= nx) s = 0.f;
+        for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
+        if (lane == 0) gmem(e.part_sq)[(int64_t)bx * pieces + p] = s;
+      }
+    }
     with_radix_a<RC>(f.a, [&](auto rc) {
       constexpr int R = decltype(rc)::value;
       float2 v[R];

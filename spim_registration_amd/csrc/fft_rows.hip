@@ -376,4 +376,73 @@ hipError_t launch_rows(int kind, int cls, const void* items, const int* prefix, 
   return hipGetLastError();
 }
 
+// ---------------------------------------------------------------------------
+// energies of what an iteration transforms
+
+__global__ __launch_bounds__(256) void k_rows_energy(const float* img, int nx, int nrows, int per, float* part) {
+  const int row0 = blockIdx.x * per, rows = min(per, nrows - row0), pieces = energy_pieces(nx);
+  const int lane = threadIdx.x & 63;
+  for (int p = threadIdx.x >> 6; p < pieces; p += 4) {
+    const int x = p * kEnergyPiece + lane;
+    const auto src = gmem(img) + (int64_t)row0 * nx + x;
+    float s = 0.f;
+    if (x < nx)
+      for (int r = 0; r < rows; ++r) {
+        const float v = src[(int64_t)r * nx];
+        s += v * v;
+      }
+    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
+    if (lane == 0) gmem(part)[(int64_t)blockIdx.x * pieces + p] = s;
+  }
+}
+
+constexpr int kEnergyThreads = 256;
+
+// A workgroup per slice of a convolution's partials, four loads in flight per
+// thread.
+__global__ __launch_bounds__(kEnergyThreads) void k_energy_sums(const EnergyItem* items) {
+  __shared__ double rs[kEnergyThreads];
+  const EnergyItem E = items[blockIdx.z];
+  const int slice = blockIdx.x, conv = blockIdx.y;
+  if (conv >= E.convs) return;  // uniform
+  const int n = E.nwg * E.pieces;
+  const int lo = (int)((int64_t)n * slice / kEnergySlices), hi = (int)((int64_t)n * (slice + 1) / kEnergySlices);
+  const auto part = gmem(E.part) + (int64_t)conv * n;
+  double s = 0.0;
+#pragma unroll 4
+  for (int i = lo + threadIdx.x; i < hi; i += kEnergyThreads) s += (double)part[i];
+  rs[threadIdx.x] = s;
+  __syncthreads();
+  for (int o = kEnergyThreads / 2; o > 0; o >>= 1) {
+    if (threadIdx.x < o) rs[threadIdx.x] += rs[threadIdx.x + o];
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) gmem(E.sums)[conv * kEnergySlices + slice] = rs[0];
+}
+
+__global__ __launch_bounds__(kEnergyThreads) void k_energy_check(const EnergyItem* items) {
+  const EnergyItem E = items[blockIdx.x];
+  int refuse = 0;
+  for (int i = threadIdx.x; i < E.convs * kEnergySlices; i += kEnergyThreads)
+    if (!(gmem(E.sums)[i] < INFINITY)) refuse = 1;  // (squares past the largest float too)
+  refuse = __syncthreads_or(refuse);
+  if (threadIdx.x == 0) *gmem(E.refuse) = refuse;
+}
+
+hipError_t launch_rows_energy(const float* img, Int3 n, int per, float* part, hipStream_t stream) {
+  const int nrows = n.y * n.z;
+  (void)hipGetLastError();
+  hipLaunchKernelGGL(k_rows_energy, dim3((nrows + per - 1) / per), dim3(256), 0, stream, img, n.x, nrows, per, part);
+  return hipGetLastError();
+}
+
+hipError_t launch_energy_check(const EnergyItem* items, int nitems, int max_convs, hipStream_t stream) {
+  (void)hipGetLastError();
+  hipLaunchKernelGGL(k_energy_sums, dim3(kEnergySlices, max_convs, nitems), dim3(kEnergyThreads), 0, stream, items);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(k_energy_check, dim3(nitems), dim3(kEnergyThreads), 0, stream, items);
+  return hipGetLastError();
+}
+
 }  // namespace mvd

@@ -230,7 +230,15 @@ struct EpilogueArgs {
   float2* rspec = nullptr;
   int rpitch = 0;
   double* part_rsum = nullptr;
+  // kEpiQuotient and kEpiUpdate with rspec (nullable): per workgroup and piece
+  // of kEnergyPiece voxels along x, the sum over its rows of the squares of what
+  // goes on to the transform
+  float* part_sq = nullptr;
+  // kEpiUpdate with rspec (nullable): the estimate before the update is kept here
+  float* keep = nullptr;
 };
+constexpr int kEnergyPiece = 64;
+__host__ __device__ inline int energy_pieces(int nx) { return (nx + kEnergyPiece - 1) / kEnergyPiece; }
 
 // Launchers (all asynchronous on `stream`).
 hipError_t launch_x_forward(const ShapePlan& sp, const ConvGeom& g, const float* src, int gather, float2* spec,
@@ -395,6 +403,18 @@ hipError_t launch_to_slabs(const ShapePlan& sp, const float2* in, float2* out, h
 int build_rows_params(const RowsPass& d, void* out, int* gx, int* gy, int* cls, int* threads, size_t* lds);
 hipError_t launch_rows(int kind, int cls, const void* items, const int* prefix, const int* gx, int nitems, int nwg,
                        int threads, size_t lds, hipStream_t stream);
+// What the convolutions of one iteration by rows transform: the partials of
+// their energies (EpilogueArgs::part_sq, one set per convolution).
+constexpr int kEnergySlices = 32;
+struct EnergyItem {
+  const float* part;  // [convs][nwg][pieces]
+  double* sums;       // [convs][kEnergySlices]
+  int* refuse;        // set to 1 if one of them holds a NaN or an infinity, else to 0
+  int convs, nwg, pieces;
+};
+// The partials of an image, `per` rows a workgroup.
+hipError_t launch_rows_energy(const float* img, Int3 n, int per, float* part, hipStream_t stream);
+hipError_t launch_energy_check(const EnergyItem* items, int nitems, int max_convs, hipStream_t stream);
 constexpr int kMaxParamBytes = 640;
 bool pass_is_fast(const PassDesc& d);
 bool pass_is_any(const PassDesc& d);

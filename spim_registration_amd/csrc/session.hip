@@ -415,6 +415,7 @@ struct PassLaunch {
   bool lines = false;  // z pass with one kernel spectrum for all items: grid (lx, ly) of lines
   int lx = 0, ly = 0;
   bool reduce = false;
+  bool energy = false;  // check of the energies of an iteration by rows; lx: convolutions of an item at most
   size_t lds = 0;
   const LaunchTables* tab = nullptr;  // uploaded before the launch
   size_t items_at = 0, prefix_at = 0, gx_at = 0;
@@ -765,7 +766,18 @@ struct mvd_session {
   // ms, of four 311x263x149 views in one window 18.7 -> 16.2 ms.  The y passes
   // run at 5.5 to 5.9 TB/s; the z pass (3.5 TB/s) and the x pass (3.6) are held
   // by VALU issue (55 %) and the latency of their three exchanges together.
+  //
+  // One value that is no finite number reaches every value of its rows, then of
+  // its tile: in block windows it reaches its blocks, in one window the image.
+  // Where those differ (`guard`), every iteration sums the squares of what its
+  // convolutions transform, and one that met a NaN or an infinity is taken back
+  // and repeated, and the later ones run, in block windows (use_windows).  The
+  // ratio image, which iterations by rows leave alone, holds the estimate
+  // meanwhile.
   struct RowConv {
+    bool guard = false;
+    DeviceBuf energy;  // partials of the squares per convolution, estimate of view 0 first
+    DeviceBuf esums;   // their sums (double), then the check's verdict (int)
     bool on = false, shared = false, consts = false;  // shared: the views' own spectra have this shape
     const ShapePlan* plan = nullptr;
     Int3 kd{0, 0, 0}, win{0, 0, 0};
@@ -791,6 +803,7 @@ struct mvd_session {
   double osem = 1.0;
   float wconst = 1.f;  // weight of every voxel without weight images
   bool prepared = false, psi_ready = false;
+  unsigned epoch = 0;  // of the buffers that launch lists name
 
   ~mvd_session() {
     if (stream) (void)hipStreamDestroy(stream);
@@ -976,6 +989,7 @@ int build_rows_launches(const std::vector<RowsPass>& passes, LaunchTables* tab, 
 
 hipError_t enqueue_pass_launch(const PassLaunch& L, hipStream_t st) {
   if (L.reduce) return launch_reduce_stats_batch(static_cast<const ReduceItem*>(L.items()), L.nitems, st);
+  if (L.energy) return launch_energy_check(static_cast<const EnergyItem*>(L.items()), L.nitems, L.lx, st);
   if (L.lines) return launch_z_lines(L.cls, L.items(), L.nitems, L.lx, L.ly, st, L.table);
   if (L.path == 2)
     return launch_batch_xy(L.kind, L.cls, L.items(), L.prefix(), L.gx(), L.nitems, L.nwg, st,
@@ -1103,7 +1117,7 @@ int rows_length(int w, int most, bool columns, double* cost) {
 // is about as cheap (within 10 %), so that the gradient uses the same spectra.
 int plan_rows(mvd_session* s) {
   auto& r = s->rc;
-  r.on = r.consts = false;
+  r.on = r.consts = r.guard = false;
   if (!g_row_conv) return 0;
   const Int3 n = s->img, kd = s->views[0].kd;
   for (auto& v : s->views)
@@ -1166,8 +1180,37 @@ int plan_rows(mvd_session* s) {
   r.geom = g;
   const int per = x_any_rows_per_wg(r.plan->px);
   r.nwg = (n.y * n.z + per - 1) / per;
+  r.guard = v0.blocks.size() > 1 || r.tiles.size() > 1;
   r.on = true;
   return 0;
+}
+
+// Where the partials of convolution `conv` (0 .. 2 nviews - 1, two of a view in
+// the order of an iteration) are.
+float* energy_of(mvd_session* s, int conv) {
+  const size_t n = (size_t)s->rc.nwg * energy_pieces(s->img.x);
+  return s->rc.energy.as<float>() + n * conv;
+}
+
+int add_energy_check(const std::vector<EnergyItem>& items, LaunchTables* tab, std::vector<PassLaunch>* out) {
+  if (items.empty()) return 0;
+  PassLaunch L;
+  L.energy = true;
+  L.timing = kTReduce;
+  L.nitems = (int)items.size();
+  for (auto& i : items) L.lx = std::max(L.lx, i.convs);
+  L.tab = tab;
+  L.items_at = tab->add(items.data(), sizeof(EnergyItem) * items.size());
+  out->push_back(std::move(L));
+  return 0;
+}
+
+// refuse: the verdict's place, or null for the session's own.
+EnergyItem energy_item(mvd_session* s, int* refuse) {
+  auto& r = s->rc;
+  const int convs = 2 * s->nviews;
+  if (!refuse) refuse = reinterpret_cast<int*>(r.esums.as<double>() + convs * kEnergySlices);
+  return {r.energy.as<float>(), r.esums.as<double>(), refuse, convs, r.nwg, energy_pieces(s->img.x)};
 }
 
 // The y and z passes and the x pass of one convolution of view v by rows.
@@ -1213,6 +1256,9 @@ void rows_pass_descs(mvd_session* s, int v, int conv, std::vector<RowsPass> (&pa
   x.e = conv_epilogue(s, v, conv, 0);
   x.e.rspec = r.rows.as<float2>();
   x.e.rpitch = r.plan->pitch;
+  // the ratio goes to the view's second convolution, the estimate to the next view's first
+  if (r.guard) x.e.part_sq = energy_of(s, conv == 0 ? 2 * v + 1 : 2 * ((v + 1) % s->nviews));
+  if (r.guard && conv == 1 && v == 0) x.e.keep = s->d_ratio.as<float>();
   xinv->push_back(x);
 }
 
@@ -1226,6 +1272,11 @@ int ensure_rows(mvd_session* s) {
   const size_t nrows = (size_t)n.y * n.z, tile_elems = slab_elems(*r.plan, n.z) * r.tiles.size();
   MVD_CHECK(r.rows.ensure(row * (nrows + 1)));
   MVD_CHECK(r.planes.ensure(sizeof(float2) * (tile_elems + slab_elems(*r.plan, 1))));
+  if (r.guard) {
+    const size_t convs = 2 * (size_t)s->nviews;
+    MVD_CHECK(r.energy.ensure(sizeof(float) * convs * r.nwg * energy_pieces(n.x)));
+    MVD_CHECK(r.esums.ensure(sizeof(double) * (convs * kEnergySlices + 1)));
+  }
   float2* crow = r.rows.as<float2>() + (size_t)r.plan->pitch * nrows;
   ConvGeom g{};
   g.src = {1, 1, 1};
@@ -1253,10 +1304,20 @@ int ensure_rows(mvd_session* s) {
   return 0;
 }
 
-// The rows of the current estimate, on stream st.
+// The rows of the current estimate, and their energies, on stream st.
 hipError_t rows_start(mvd_session* s, hipStream_t st) {
-  return launch_x_forward_any(*s->rc.plan, s->rc.geom, s->d_psi.as<float>(), kGatherMirror, s->rc.rows.as<float2>(),
-                              st);
+  auto& r = s->rc;
+  if (r.guard) {
+    const hipError_t e =
+        launch_rows_energy(s->d_psi.as<float>(), s->img, x_any_rows_per_wg(r.plan->px), energy_of(s, 0), st);
+    if (e != hipSuccess) return e;
+  }
+  return launch_x_forward_any(*r.plan, r.geom, s->d_psi.as<float>(), kGatherMirror, r.rows.as<float2>(), st);
+}
+
+// The estimate before the iteration by rows, which its first update has kept.
+hipError_t restore_psi(mvd_session* s, hipStream_t st) {
+  return hipMemcpyAsync(s->d_psi.p, s->d_ratio.p, sizeof(float) * s->n, hipMemcpyDeviceToDevice, st);
 }
 
 // Launch lists of the block-batched iteration (one spectrum buffer per block).
@@ -1279,6 +1340,9 @@ int build_block_batch(mvd_session* s) {
         for (auto& p : pass)
           if ((rc = build_rows_launches(p, &bb.tables, &bb.view[v]))) return rc;
         if ((rc = build_pass_launches(xinv, &bb.tables, &bb.view[v]))) return rc;
+        // (before the last update makes the estimate of the next iteration)
+        if (s->rc.guard && conv == 0 && v == s->nviews - 1)
+          if ((rc = add_energy_check({energy_item(s, nullptr)}, &bb.tables, &bb.view[v]))) return rc;
       }
     MVD_CHECK(bb.tables.upload());
     bb.built = bb.enabled = true;
@@ -1911,6 +1975,70 @@ int ensure_workspace(mvd_session* s) {
   return 0;
 }
 
+// Leaves the iteration by rows for good: its buffers go, the block windows'
+// spectra and workspace are made.  Nothing may run on the session's buffers.
+int use_windows(mvd_session* s) {
+  auto& r = s->rc;
+  r.on = r.consts = r.guard = false;
+  for (DeviceBuf* b : {&r.rows, &r.planes, &r.plain, &r.energy, &r.esums}) *b = DeviceBuf();
+  for (auto& v : s->views) {
+    v.r1hat = DeviceBuf();
+    v.r2hat = DeviceBuf();
+  }
+  s->bb.built = false;
+  ++s->epoch;
+  for (int v = 0; v < s->nviews; ++v) {
+    int rc = view_spectra(s, v);
+    if (rc) return rc;
+  }
+  int rc = ensure_workspace(s);
+  if (rc) return rc;
+  MVD_CHECK(hipStreamSynchronize(s->stream));
+  return 0;
+}
+
+// One iteration on the session's stream, its statistics to the it-th place of d_stats.
+int enqueue_iteration(mvd_session* s, int it) {
+  double* stats = s->d_stats.as<double>() + 2 * (size_t)it * s->nviews;
+  // blocks of a view together: per pass one launch for all blocks
+  for (int v = 0; s->bb.enabled && v < s->nviews; ++v) {
+    for (auto& L : s->bb.view[v]) {
+      s->timer.begin(s->stream);
+      MVD_CHECK(enqueue_pass_launch(L, s->stream));
+      s->timer.end(s->stream, L.timing);
+    }
+    s->timer.begin(s->stream);
+    MVD_CHECK(launch_reduce_stats(s->d_part_sum.as<double>(), s->d_part_max.as<float>(),
+                                  s->rc.on ? s->rc.nwg : s->views[v].nwg_update, stats + 2 * v, s->stream));
+    s->timer.end(s->stream, kTReduce);
+  }
+  // block after block through one spectrum buffer
+  float2* spec = s->d_spec.as<float2>();
+  for (int v = 0; !s->bb.enabled && v < s->nviews; ++v) {
+    auto& view = s->views[v];
+    const ShapePlan& sp = *view.plan;
+    // convolve1 + quotient: psi -> ratio (MVDeconvolution.java:383-406)
+    const EpilogueArgs q = conv_epilogue(s, v, 0, 0);
+    for (auto& g : view.blocks) {
+      int rc = run_conv(s, sp, g, s->d_psi.as<float>(), kGatherMirror, view.k1hat.as<float2>(), q, spec);
+      if (rc) return rc;
+    }
+    // convolve2 + update: ratio -> psi (MVDeconvolution.java:418-457)
+    int off = 0;
+    for (auto& g : view.blocks) {
+      const EpilogueArgs u = conv_epilogue(s, v, 1, off);
+      int rc = run_conv(s, sp, g, s->d_ratio.as<float>(), kGatherOne, view.k2hat.as<float2>(), u, spec);
+      if (rc) return rc;
+      off += conv_inverse_workgroups(sp, g);
+    }
+    s->timer.begin(s->stream);
+    MVD_CHECK(launch_reduce_stats(s->d_part_sum.as<double>(), s->d_part_max.as<float>(), off, stats + 2 * v,
+                                  s->stream));
+    s->timer.end(s->stream, kTReduce);
+  }
+  return 0;
+}
+
 constexpr int kReduceParts = 2048;
 
 // Sum of the per-voxel means and number of voxels with data (FirstIteration).
@@ -2160,6 +2288,7 @@ int mvd_prepare(mvd_session* s, int psf_type, double lambda, const int* block_xy
   int rc = ensure_workspace(s);
   if (rc) return rc;
   MVD_CHECK(hipStreamSynchronize(s->stream));
+  ++s->epoch;
   s->prepared = true;
   return 0;
 }
@@ -2256,12 +2385,6 @@ int mvd_iterate(mvd_session* s, int n, double* stats) {
   if (n == 0) return 0;
   DeviceGuard guard(s->device);
   MVD_CHECK(s->d_stats.ensure(sizeof(double) * 2 * s->nviews * (size_t)n));
-  float* psi = s->d_psi.as<float>();
-  float* ratio = s->d_ratio.as<float>();
-  float2* spec = s->d_spec.as<float2>();
-  const int wm = s->weight_mode == MVD_WEIGHTS_NONE ? kWeightNone
-                 : s->weight_mode == MVD_WEIGHTS_VIRTUAL ? kWeightVirtual
-                                                         : kWeightArray;
   if (!s->bb.built) {
     int rc = build_block_batch(s);
     if (rc) return rc;
@@ -2271,58 +2394,17 @@ int mvd_iterate(mvd_session* s, int n, double* stats) {
     MVD_CHECK(rows_start(s, s->stream));
     s->timer.end(s->stream, kTXForward);
   }
-  // blocks of a view together: per pass one launch for all blocks
-  for (int it = 0; s->bb.enabled && it < n; ++it) {
-    for (int v = 0; v < s->nviews; ++v) {
-      for (auto& L : s->bb.view[v]) {
-        s->timer.begin(s->stream);
-        MVD_CHECK(enqueue_pass_launch(L, s->stream));
-        s->timer.end(s->stream, L.timing);
-      }
-      s->timer.begin(s->stream);
-      MVD_CHECK(launch_reduce_stats(s->d_part_sum.as<double>(), s->d_part_max.as<float>(),
-                                    s->rc.on ? s->rc.nwg : s->views[v].nwg_update,
-                                    s->d_stats.as<double>() + 2 * ((size_t)it * s->nviews + v), s->stream));
-      s->timer.end(s->stream, kTReduce);
-    }
-  }
-  // block after block through one spectrum buffer
-  for (int it = 0; !s->bb.enabled && it < n; ++it) {
-    for (int v = 0; v < s->nviews; ++v) {
-      auto& view = s->views[v];
-      const ShapePlan& sp = *view.plan;
-      // convolve1 + quotient: psi -> ratio (MVDeconvolution.java:383-406)
-      EpilogueArgs q{};
-      q.mode = kEpiQuotient;
-      q.dst = ratio;
-      q.img = s->d_views.as<float>() + v * s->n;
-      for (auto& g : view.blocks) {
-        int rc = run_conv(s, sp, g, psi, kGatherMirror, view.k1hat.as<float2>(), q, spec);
-        if (rc) return rc;
-      }
-      // convolve2 + update: ratio -> psi (MVDeconvolution.java:418-457)
-      EpilogueArgs u{};
-      u.mode = kEpiUpdate;
-      u.dst = psi;
-      u.weight_mode = wm;
-      u.weight = wm == kWeightNone ? nullptr : s->d_weights.as<float>() + v * s->n;
-      u.wsum = s->d_wsum.as<float>();
-      u.osem = s->osem;
-      u.wconst = s->wconst;
-      u.lambda = s->lambda;
-      int off = 0;
-      for (auto& g : view.blocks) {
-        u.part_sum = s->d_part_sum.as<double>() + off;
-        u.part_max = s->d_part_max.as<float>() + off;
-        int rc = run_conv(s, sp, g, ratio, kGatherOne, view.k2hat.as<float2>(), u, spec);
-        if (rc) return rc;
-        off += conv_inverse_workgroups(sp, g);
-      }
-      s->timer.begin(s->stream);
-      MVD_CHECK(launch_reduce_stats(s->d_part_sum.as<double>(), s->d_part_max.as<float>(), off,
-                                    s->d_stats.as<double>() + 2 * ((size_t)it * s->nviews + v), s->stream));
-      s->timer.end(s->stream, kTReduce);
-    }
+  for (int it = 0; it < n; ++it) {
+    const bool guard = s->rc.on && s->rc.guard;
+    int rc = enqueue_iteration(s, it);
+    if (rc) return rc;
+    if (!guard) continue;
+    int refuse = 0;
+    MVD_CHECK(hipMemcpyAsync(&refuse, energy_item(s, nullptr).refuse, sizeof(int), hipMemcpyDeviceToHost, s->stream));
+    MVD_CHECK(hipStreamSynchronize(s->stream));
+    if (!refuse) continue;
+    MVD_CHECK(restore_psi(s, s->stream));
+    if ((rc = use_windows(s)) || (rc = build_block_batch(s)) || (rc = enqueue_iteration(s, it))) return rc;
   }
   if (stats)
     MVD_CHECK(hipMemcpyAsync(stats, s->d_stats.p, sizeof(double) * 2 * s->nviews * (size_t)n,
@@ -2799,7 +2881,9 @@ struct mvd_batch {
   std::vector<PassLaunch> launches;
   LaunchTables tables;
   DeviceBuf stats_iter, stats_hist;
+  DeviceBuf refuse;  // per stack, the verdict of its iteration by rows
   std::vector<int> stats_off;  // per stack, in doubles
+  std::vector<unsigned> epoch;  // per stack, of the launches
   int total_stats = 0;
   bool prepared = false, use_graph = false;
   hipGraph_t graph = nullptr;
@@ -2815,6 +2899,127 @@ namespace {
 
 int enqueue_batch_iteration(mvd_batch* b) {
   for (auto& L : b->launches) MVD_CHECK(enqueue_pass_launch(L, b->stream));
+  return 0;
+}
+
+// Launches (and the graph) of a batch's iteration.
+int build_batch(mvd_batch* b) {
+  b->prepared = false;
+  if (b->exec) (void)hipGraphExecDestroy(b->exec);
+  if (b->graph) (void)hipGraphDestroy(b->graph);
+  b->exec = nullptr;
+  b->graph = nullptr;
+  b->launches.clear();
+  b->tables.host.clear();
+  b->spec.clear();
+  b->stats_off.clear();
+  b->epoch.clear();
+  MVD_CHECK(b->refuse.ensure(sizeof(int) * b->stacks.size()));
+  int maxv = 0, tot = 0;
+  for (auto* s : b->stacks) {
+    MVD_REQUIRE(s->prepared, "a session is not prepared");
+    b->stats_off.push_back(tot);
+    tot += 2 * s->nviews;
+    maxv = std::max(maxv, s->nviews);
+    size_t nb = 0;
+    for (auto& v : s->views) nb = std::max(nb, v.blocks.size());
+    b->epoch.push_back(s->epoch);
+    b->spec.emplace_back();
+    if (s->rc.on) {
+      int rc = ensure_rows(s);
+      if (rc) return rc;
+      continue;
+    }
+    for (size_t i = 0; i < nb; ++i) {
+      b->spec.back().emplace_back();
+      size_t elems = 0;
+      for (auto& v : s->views)
+        if (i < v.blocks.size()) elems = std::max<size_t>(elems, v.plan->spectrum_elems());
+      MVD_CHECK(b->spec.back().back().ensure(sizeof(float2) * elems));
+      // finite row padding (before any capture)
+      MVD_CHECK(hipMemsetAsync(b->spec.back().back().p, 0, sizeof(float2) * elems, b->stream));
+    }
+  }
+  b->total_stats = tot;
+  MVD_CHECK(b->stats_iter.ensure(sizeof(double) * tot));
+  for (int v = 0; v < maxv; ++v) {
+    for (int conv = 0; conv < 2; ++conv) {
+      std::vector<PassDesc> pass[5];
+      std::vector<RowsPass> rows[3];
+      for (size_t si = 0; si < b->stacks.size(); ++si) {
+        mvd_session* s = b->stacks[si];
+        if (v >= s->nviews) continue;
+        if (s->rc.on) {
+          rows_pass_descs(s, v, conv, rows, &pass[4]);
+          continue;
+        }
+        std::vector<float2*> spec;
+        for (auto& buf : b->spec[si]) spec.push_back(buf.as<float2>());
+        conv_pass_descs(s, v, conv, spec, pass);
+      }
+      for (int p = 0; p < 5; ++p) {
+        if (p > 0 && p < 4)
+          if (int rc = build_rows_launches(rows[p - 1], &b->tables, &b->launches)) return rc;
+        int rc = build_pass_launches(pass[p], &b->tables, &b->launches);
+        if (rc) return rc;
+      }
+      if (conv == 0) {
+        std::vector<EnergyItem> checks;
+        for (size_t si = 0; si < b->stacks.size(); ++si)
+          if (b->stacks[si]->rc.guard && v == b->stacks[si]->nviews - 1)
+            checks.push_back(energy_item(b->stacks[si], b->refuse.as<int>() + si));
+        if (int rc = add_energy_check(checks, &b->tables, &b->launches)) return rc;
+      }
+    }
+    // statistics of view slot v
+    std::vector<ReduceItem> red;
+    for (size_t si = 0; si < b->stacks.size(); ++si) {
+      mvd_session* s = b->stacks[si];
+      if (v >= s->nviews) continue;
+      int n = 0;
+      for (auto& g : s->views[v].blocks) n += conv_inverse_workgroups(*s->views[v].plan, g);
+      if (s->rc.on) n = s->rc.nwg;
+      red.push_back({s->d_part_sum.as<double>(), s->d_part_max.as<float>(), n,
+                     b->stats_iter.as<double>() + b->stats_off[si] + 2 * v});
+    }
+    PassLaunch L;
+    L.reduce = true;
+    L.timing = kTReduce;
+    L.nitems = (int)red.size();
+    L.tab = &b->tables;
+    L.items_at = b->tables.add(red.data(), sizeof(ReduceItem) * red.size());
+    b->launches.push_back(std::move(L));
+  }
+  MVD_CHECK(b->tables.upload());
+  if (b->use_graph) {
+    MVD_CHECK(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
+    int rc = enqueue_batch_iteration(b);
+    hipGraph_t g = nullptr;
+    hipError_t ec = hipStreamEndCapture(b->stream, &g);
+    if (rc) {
+      if (g) (void)hipGraphDestroy(g);
+      return rc;
+    }
+    MVD_CHECK(ec);
+    b->graph = g;
+    MVD_CHECK(hipGraphInstantiate(&b->exec, b->graph, nullptr, nullptr, 0));
+  }
+  b->prepared = true;
+  return 0;
+}
+
+// The it-th iteration of stack si once more, in block windows and by itself.
+int repeat_in_windows(mvd_batch* b, size_t si, int it) {
+  mvd_session* s = b->stacks[si];
+  MVD_CHECK(restore_psi(s, s->stream));
+  MVD_CHECK(s->d_stats.ensure(sizeof(double) * 2 * s->nviews));
+  int rc;
+  if ((rc = use_windows(s)) || (rc = build_block_batch(s)) || (rc = enqueue_iteration(s, 0))) return rc;
+  MVD_CHECK(hipMemcpyAsync(b->stats_hist.as<double>() + (size_t)it * b->total_stats + b->stats_off[si], s->d_stats.p,
+                           sizeof(double) * 2 * s->nviews, hipMemcpyDeviceToDevice, s->stream));
+  MVD_CHECK(hipStreamSynchronize(s->stream));
+  s->timer.collect();
+  s->bb = mvd_session::BlockBatch();  // (the batch has block spectra of its own)
   return 0;
 }
 
@@ -2858,98 +3063,8 @@ int mvd_batch_prepare(mvd_batch* b, int use_graph) {
   MVD_REQUIRE(b, "NULL batch");
   MVD_REQUIRE(!b->stacks.empty(), "no sessions in the batch");
   DeviceGuard guard(b->device);
-  if (b->exec) (void)hipGraphExecDestroy(b->exec);
-  if (b->graph) (void)hipGraphDestroy(b->graph);
-  b->exec = nullptr;
-  b->graph = nullptr;
-  b->launches.clear();
-  b->tables.host.clear();
-  b->spec.clear();
-  b->stats_off.clear();
-  int maxv = 0, tot = 0;
-  for (auto* s : b->stacks) {
-    MVD_REQUIRE(s->prepared, "a session is not prepared");
-    b->stats_off.push_back(tot);
-    tot += 2 * s->nviews;
-    maxv = std::max(maxv, s->nviews);
-    size_t nb = 0;
-    for (auto& v : s->views) nb = std::max(nb, v.blocks.size());
-    b->spec.emplace_back();
-    if (s->rc.on) {
-      int rc = ensure_rows(s);
-      if (rc) return rc;
-      continue;
-    }
-    for (size_t i = 0; i < nb; ++i) {
-      b->spec.back().emplace_back();
-      size_t elems = 0;
-      for (auto& v : s->views)
-        if (i < v.blocks.size()) elems = std::max<size_t>(elems, v.plan->spectrum_elems());
-      MVD_CHECK(b->spec.back().back().ensure(sizeof(float2) * elems));
-      // finite row padding (before any capture)
-      MVD_CHECK(hipMemsetAsync(b->spec.back().back().p, 0, sizeof(float2) * elems, b->stream));
-    }
-  }
-  b->total_stats = tot;
-  MVD_CHECK(b->stats_iter.ensure(sizeof(double) * tot));
-  for (int v = 0; v < maxv; ++v) {
-    for (int conv = 0; conv < 2; ++conv) {
-      std::vector<PassDesc> pass[5];
-      std::vector<RowsPass> rows[3];
-      for (size_t si = 0; si < b->stacks.size(); ++si) {
-        mvd_session* s = b->stacks[si];
-        if (v >= s->nviews) continue;
-        if (s->rc.on) {
-          rows_pass_descs(s, v, conv, rows, &pass[4]);
-          continue;
-        }
-        std::vector<float2*> spec;
-        for (auto& buf : b->spec[si]) spec.push_back(buf.as<float2>());
-        conv_pass_descs(s, v, conv, spec, pass);
-      }
-      for (int p = 0; p < 5; ++p) {
-        if (p > 0 && p < 4)
-          if (int rc = build_rows_launches(rows[p - 1], &b->tables, &b->launches)) return rc;
-        int rc = build_pass_launches(pass[p], &b->tables, &b->launches);
-        if (rc) return rc;
-      }
-    }
-    // statistics of view slot v
-    std::vector<ReduceItem> red;
-    for (size_t si = 0; si < b->stacks.size(); ++si) {
-      mvd_session* s = b->stacks[si];
-      if (v >= s->nviews) continue;
-      int n = 0;
-      for (auto& g : s->views[v].blocks) n += conv_inverse_workgroups(*s->views[v].plan, g);
-      if (s->rc.on) n = s->rc.nwg;
-      red.push_back({s->d_part_sum.as<double>(), s->d_part_max.as<float>(), n,
-                     b->stats_iter.as<double>() + b->stats_off[si] + 2 * v});
-    }
-    PassLaunch L;
-    L.reduce = true;
-    L.timing = kTReduce;
-    L.nitems = (int)red.size();
-    L.tab = &b->tables;
-    L.items_at = b->tables.add(red.data(), sizeof(ReduceItem) * red.size());
-    b->launches.push_back(std::move(L));
-  }
-  MVD_CHECK(b->tables.upload());
   b->use_graph = use_graph != 0;
-  if (b->use_graph) {
-    MVD_CHECK(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
-    int rc = enqueue_batch_iteration(b);
-    hipGraph_t g = nullptr;
-    hipError_t ec = hipStreamEndCapture(b->stream, &g);
-    if (rc) {
-      if (g) (void)hipGraphDestroy(g);
-      return rc;
-    }
-    MVD_CHECK(ec);
-    b->graph = g;
-    MVD_CHECK(hipGraphInstantiate(&b->exec, b->graph, nullptr, nullptr, 0));
-  }
-  b->prepared = true;
-  return 0;
+  return build_batch(b);
 }
 
 int mvd_batch_iterate(mvd_batch* b, int n, double* stats) {
@@ -2959,10 +3074,19 @@ int mvd_batch_iterate(mvd_batch* b, int n, double* stats) {
   for (auto* s : b->stacks) MVD_REQUIRE(s->psi_ready, "mvd_init_psi every session first");
   if (n == 0) return 0;
   DeviceGuard guard(b->device);
+  // (a stack that was prepared again, or has left the iteration by rows, has other buffers)
+  for (size_t si = 0; si < b->stacks.size(); ++si)
+    if (b->epoch[si] != b->stacks[si]->epoch) {
+      int rc = build_batch(b);
+      if (rc) return rc;
+      break;
+    }
   MVD_CHECK(b->stats_hist.ensure(sizeof(double) * (size_t)b->total_stats * n));
   for (auto* s : b->stacks)
     if (s->rc.on) MVD_CHECK(rows_start(s, b->stream));
   for (int it = 0; it < n; ++it) {
+    bool guard = false;
+    for (auto* s : b->stacks) guard = guard || s->rc.guard;
     if (b->use_graph) {
       MVD_CHECK(hipGraphLaunch(b->exec, b->stream));
     } else {
@@ -2971,6 +3095,20 @@ int mvd_batch_iterate(mvd_batch* b, int n, double* stats) {
     }
     MVD_CHECK(hipMemcpyAsync(b->stats_hist.as<double>() + (size_t)it * b->total_stats, b->stats_iter.p,
                              sizeof(double) * b->total_stats, hipMemcpyDeviceToDevice, b->stream));
+    if (!guard) continue;
+    std::vector<int> refuse(b->stacks.size());
+    MVD_CHECK(hipMemcpyAsync(refuse.data(), b->refuse.p, sizeof(int) * refuse.size(), hipMemcpyDeviceToHost,
+                             b->stream));
+    MVD_CHECK(hipStreamSynchronize(b->stream));
+    bool left = false;
+    for (size_t si = 0; si < b->stacks.size(); ++si)
+      if (b->stacks[si]->rc.guard && refuse[si]) {
+        left = true;
+        int rc = repeat_in_windows(b, si, it);
+        if (rc) return rc;
+      }
+    if (left && it + 1 < n)
+      if (int rc = build_batch(b)) return rc;
   }
   if (stats)
     MVD_CHECK(hipMemcpyAsync(stats, b->stats_hist.p, sizeof(double) * (size_t)b->total_stats * n,
