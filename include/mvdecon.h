@@ -232,6 +232,14 @@ int mvd_set_weights(mvd_session* s, int mode, int osem_index, double osem_value,
  * whose FFT sizes are chosen by its FFT library. */
 int mvd_set_fft_policy(mvd_session* s, int policy);
 
+/* on != 0: the iterations use the block windows whatever the kernels
+ * (call before mvd_prepare). */
+int mvd_set_block_windows(mvd_session* s, int on);
+
+/* 1 if the next iteration runs by rows, 0 in block windows (after mvd_prepare;
+ * a session can change from rows to windows at an iteration). */
+int mvd_by_rows(mvd_session* s);
+
 /* MVDeconInput.init(PSFTYPE) (deconv/MVDeconInput.java:62-68 -> MVDeconFFT.init,
  * deconv/MVDeconFFT.java:183-324) plus block split.  block_xyz NULL = the whole
  * image as one block of img+k-1 (MVDeconFFT.java:144-165); otherwise

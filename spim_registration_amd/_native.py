@@ -25,7 +25,7 @@ EXPORTS = (
     "mvd_set_weights", "mvd_prepare", "mvd_init_psi",
     "mvd_iterate", "mvd_get_psi", "mvd_get_kernels", "mvd_set_psf", "mvd_set_psfs", "mvd_psi_sum", "mvd_set_timing", "mvd_get_timing",
     "mvd_timing_name", "mvd_get_geometry", "mvd_last_error", "mvd_nll_grad", "mvd_nll_grad_device",
-    "mvd_get_grad_psi", "mvd_set_fft_policy",
+    "mvd_get_grad_psi", "mvd_set_fft_policy", "mvd_set_block_windows", "mvd_by_rows",
     "mvd_min_max", "mvd_min_max_device", "mvd_u16_range", "mvd_convert_u16_device", "mvd_write_tiff",
     "mvd_export_psi",
     "mvd_batch_create", "mvd_batch_add", "mvd_batch_prepare", "mvd_batch_iterate", "mvd_batch_destroy",
@@ -101,6 +101,8 @@ def _declare(L):
     L.mvd_nll_grad_device.argtypes = [_P, _P, _P, _P, ctypes.c_int, _P]
     L.mvd_get_grad_psi.argtypes = [_P, _P]
     L.mvd_set_fft_policy.argtypes = [_P, ctypes.c_int]
+    L.mvd_set_block_windows.argtypes = [_P, ctypes.c_int]
+    L.mvd_by_rows.argtypes = [_P]
     L.mvd_batch_create.argtypes = [ctypes.c_int, _P]
     L.mvd_batch_add.argtypes = [_P, _P]
     L.mvd_batch_prepare.argtypes = [_P, ctypes.c_int]

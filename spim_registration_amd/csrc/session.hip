@@ -453,13 +453,6 @@ static const bool g_grad_keep_w = [] {
   return !(v && v[0] == '0');
 }();
 
-// MVD_ROW_CONV=0: the iteration convolves the blocks one window each
-// (comparisons).
-static const bool g_row_conv = [] {
-  const char* v = std::getenv("MVD_ROW_CONV");
-  return !(v && v[0] == '0');
-}();
-
 static int mirror_single_host(int p, int n) {
   if (p >= 0 && p < n) return p;
   if (n == 1) return 0;
@@ -803,6 +796,7 @@ struct mvd_session {
   double osem = 1.0;
   float wconst = 1.f;  // weight of every voxel without weight images
   bool prepared = false, psi_ready = false;
+  bool windows_only = false;  // mvd_set_block_windows
   unsigned epoch = 0;  // of the buffers that launch lists name
 
   ~mvd_session() {
@@ -1118,7 +1112,7 @@ int rows_length(int w, int most, bool columns, double* cost) {
 int plan_rows(mvd_session* s) {
   auto& r = s->rc;
   r.on = r.consts = r.guard = false;
-  if (!g_row_conv) return 0;
+  if (s->windows_only) return 0;
   const Int3 n = s->img, kd = s->views[0].kd;
   for (auto& v : s->views)
     if (v.kd.x != kd.x || v.kd.y != kd.y || v.kd.z != kd.z) return 0;
@@ -2300,6 +2294,15 @@ int mvd_set_fft_policy(mvd_session* s, int policy) {
   s->prepared = false;
   return 0;
 }
+
+int mvd_set_block_windows(mvd_session* s, int on) {
+  MVD_REQUIRE(s, "NULL session");
+  s->windows_only = on != 0;
+  s->prepared = false;
+  return 0;
+}
+
+int mvd_by_rows(mvd_session* s) { return s && s->prepared && s->rc.on ? 1 : 0; }
 
 int mvd_set_psf(mvd_session* s, int view, const float* psf) {
   MVD_REQUIRE(s && psf, "NULL argument");

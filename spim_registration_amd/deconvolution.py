@@ -225,14 +225,15 @@ class MVDeconvolution:
     """MVDeconvolution (MVDeconvolution.java:94-211): the constructor runs the
     whole deconvolution, like the reference; `get_psi()` returns the masked
     estimate.  `run=False` only prepares (kernels, initial estimate) so that
-    `run_iteration()` can be driven step by step."""
+    `run_iteration()` can be driven step by step.  `block_windows=True` keeps
+    the iterations in block windows (mvd_set_block_windows)."""
 
     min_value = np.float32(0.0001)
 
     def __init__(self, views: MVDeconInput, iteration_type: PSFTYPE, num_iterations: int, lam: float,
                  osem_speedup: float = 1.0, osem_speedup_index: int = 0, name: str = "deconvolved",
                  norm_threads: int = 8, weight_type: Optional[WeightType] = None,
-                 initial_psi=None, run: bool = True, fft_policy: int = 0):
+                 initial_psi=None, run: bool = True, fft_policy: int = 0, block_windows: bool = False):
         vs = views.get_views()
         if not vs:
             raise ValueError("no views")
@@ -266,6 +267,7 @@ class MVDeconvolution:
                                         float(osem_speedup), int(norm_threads), mm), "mvd_set_weights")
         self.min_overlapping_views, self.avg_overlapping_views = mm[0], mm[1]
         _native.check(L.mvd_set_fft_policy(self._s.handle, int(fft_policy)), "mvd_set_fft_policy")
+        _native.check(L.mvd_set_block_windows(self._s.handle, 1 if block_windows else 0), "mvd_set_block_windows")
         blk = None
         if v0.use_blocks:
             blk = (ctypes.c_int * 3)(*v0.block_size)
@@ -311,6 +313,11 @@ class MVDeconvolution:
         g = (ctypes.c_int * 4)()
         _native.check(_native.lib().mvd_get_geometry(self._s.handle, view, g), "mvd_get_geometry")
         return dict(blocks=g[0], fft=(g[1], g[2], g[3]))
+
+    @property
+    def by_rows(self) -> bool:
+        """Whether the next iteration runs by rows (else in block windows)."""
+        return _native.lib().mvd_by_rows(self._s.handle) == 1
 
     def nll_grad(self, psi=None, psfs=None, want_psi: bool = True, want_psf: bool = True,
                  psi_on_device: bool = False):
