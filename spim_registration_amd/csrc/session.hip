@@ -1103,6 +1103,17 @@ int rows_length(int w, int most, bool columns, double* cost) {
   return best;
 }
 
+// No iteration by rows until the next mvd_prepare; its buffers go.
+void drop_rows(mvd_session* s) {
+  auto& r = s->rc;
+  r.on = r.consts = r.guard = false;
+  for (DeviceBuf* b : {&r.rows, &r.planes, &r.plain, &r.energy, &r.esums}) *b = DeviceBuf();
+  for (auto& v : s->views) {
+    v.r1hat = DeviceBuf();
+    v.r2hat = DeviceBuf();
+  }
+}
+
 // Chooses the whole-image iteration of a prepared session (RowConv): needs one
 // kernel size for all views (they share the rows), lengths with two-radix
 // kernels, and its buffers in half of the free memory; otherwise the blocks are
@@ -1176,6 +1187,15 @@ int plan_rows(mvd_session* s) {
   r.nwg = (n.y * n.z + per - 1) / per;
   r.guard = v0.blocks.size() > 1 || r.tiles.size() > 1;
   r.on = true;
+  if (r.shared) return 0;
+  // the kernels' spectra now, the rest at the first iteration (reserve_rows)
+  bool have_mem = r.plain.ensure(sizeof(float2) * r.plan->spectrum_elems()) == hipSuccess;
+  for (auto& v : s->views)
+    have_mem = have_mem && v.r1hat.ensure(spec_b) == hipSuccess && v.r2hat.ensure(spec_b) == hipSuccess;
+  if (!have_mem) {
+    (void)hipGetLastError();
+    drop_rows(s);
+  }
   return 0;
 }
 
@@ -1256,21 +1276,34 @@ void rows_pass_descs(mvd_session* s, int v, int conv, std::vector<RowsPass> (&pa
   xinv->push_back(x);
 }
 
-// Buffers of the iteration by rows, and the spectra of the constant one that
-// the ratio has outside the image: a row along x, a plane along x and y.
+// Buffers of the iteration by rows.  They are allocated at the first iteration
+// (a session may never iterate), when the memory that plan_rows saw may be
+// gone: false, and the caller goes on in block windows.
+bool reserve_rows(mvd_session* s) {
+  auto& r = s->rc;
+  if (r.consts) return true;
+  const Int3 n = s->img;
+  const size_t nrows = (size_t)n.y * n.z, convs = r.guard ? 2 * (size_t)s->nviews : 0;
+  const std::pair<DeviceBuf*, size_t> sizes[] = {
+      {&r.rows, sizeof(float2) * r.plan->pitch * (nrows + 1)},
+      {&r.planes, sizeof(float2) * (slab_elems(*r.plan, n.z) * r.tiles.size() + slab_elems(*r.plan, 1))},
+      {&r.energy, sizeof(float) * convs * r.nwg * energy_pieces(n.x)},
+      {&r.esums, r.guard ? sizeof(double) * (convs * kEnergySlices + 1) : 0}};
+  for (auto& b : sizes)
+    if (b.first->ensure(b.second) != hipSuccess) {
+      (void)hipGetLastError();
+      return false;
+    }
+  return true;
+}
+
+// The spectra of the constant one that the ratio has outside the image: a row
+// along x, a plane along x and y.  After reserve_rows.
 int ensure_rows(mvd_session* s) {
   auto& r = s->rc;
   if (r.consts) return 0;
   const Int3 n = s->img, q = r.plan->q;
-  const size_t row = sizeof(float2) * (size_t)r.plan->pitch;
   const size_t nrows = (size_t)n.y * n.z, tile_elems = slab_elems(*r.plan, n.z) * r.tiles.size();
-  MVD_CHECK(r.rows.ensure(row * (nrows + 1)));
-  MVD_CHECK(r.planes.ensure(sizeof(float2) * (tile_elems + slab_elems(*r.plan, 1))));
-  if (r.guard) {
-    const size_t convs = 2 * (size_t)s->nviews;
-    MVD_CHECK(r.energy.ensure(sizeof(float) * convs * r.nwg * energy_pieces(n.x)));
-    MVD_CHECK(r.esums.ensure(sizeof(double) * (convs * kEnergySlices + 1)));
-  }
   float2* crow = r.rows.as<float2>() + (size_t)r.plan->pitch * nrows;
   ConvGeom g{};
   g.src = {1, 1, 1};
@@ -1314,11 +1347,15 @@ hipError_t restore_psi(mvd_session* s, hipStream_t st) {
   return hipMemcpyAsync(s->d_psi.p, s->d_ratio.p, sizeof(float) * s->n, hipMemcpyDeviceToDevice, st);
 }
 
+int use_windows(mvd_session* s);
+
 // Launch lists of the block-batched iteration (one spectrum buffer per block).
 // Off for single-block views and when the extra spectra would take more than
 // half of the free device memory.
 int build_block_batch(mvd_session* s) {
   auto& bb = s->bb;
+  if (s->rc.on && !reserve_rows(s))
+    if (int rc = use_windows(s)) return rc;
   bb.view.clear();
   bb.ztab.clear();
   bb.tables.host.clear();
@@ -1972,13 +2009,7 @@ int ensure_workspace(mvd_session* s) {
 // Leaves the iteration by rows for good: its buffers go, the block windows'
 // spectra and workspace are made.  Nothing may run on the session's buffers.
 int use_windows(mvd_session* s) {
-  auto& r = s->rc;
-  r.on = r.consts = r.guard = false;
-  for (DeviceBuf* b : {&r.rows, &r.planes, &r.plain, &r.energy, &r.esums}) *b = DeviceBuf();
-  for (auto& v : s->views) {
-    v.r1hat = DeviceBuf();
-    v.r2hat = DeviceBuf();
-  }
+  drop_rows(s);
   s->bb.built = false;
   ++s->epoch;
   for (int v = 0; v < s->nviews; ++v) {
@@ -2921,6 +2952,8 @@ int build_batch(mvd_batch* b) {
   int maxv = 0, tot = 0;
   for (auto* s : b->stacks) {
     MVD_REQUIRE(s->prepared, "a session is not prepared");
+    if (s->rc.on && !reserve_rows(s))
+      if (int rc = use_windows(s)) return rc;
     b->stats_off.push_back(tot);
     tot += 2 * s->nviews;
     maxv = std::max(maxv, s->nviews);
