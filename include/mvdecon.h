@@ -158,11 +158,18 @@ int mvd_psf_transform_size(const int* psf_size, const double* model, int* new_si
 
 /* FFT shape of each block window (call before mvd_prepare).  The iteration of a
  * session whose views have kernels of one size runs over the whole image by
- * rows in a shape of its own, whatever the blocks (blocked and whole
- * convolutions are one operator; only rounding differs); the gradient, and
- * sessions that it does not take (kernels of several sizes, arrays of 4 GiB or
- * more, buffers past half of the free memory), use the block windows.
- * mvd_get_geometry reports the block windows. */
+ * rows in a shape of its own, whatever the blocks.  Blocked and whole
+ * convolutions are one operator on finite numbers, but not in what a NaN or an
+ * infinity reaches, nor in rounding where a part of the image is much brighter
+ * than the rest.  So a session of several blocks checks every iteration: one
+ * that meets such a value, or a block whose mean square is small against the
+ * image's (of its deviation from the views' mean), is repeated in the block
+ * windows, where the session then stays until the next mvd_prepare.  By rows no
+ * block is further from 64 bits than in its window.  The gradient, and sessions
+ * that rows do not take (kernels of several sizes, blocks of less than 64
+ * voxels along x, arrays of 4 GiB or more, buffers past half of the free
+ * memory or not to be had), use the block windows.  mvd_get_geometry reports
+ * the block windows, mvd_by_rows the path. */
 enum {
   MVD_FFT_SMOOTH = 0,   /* smallest 5-smooth size per axis (default) */
   MVD_FFT_POW2 = 1,     /* smallest power of two per axis (up to 1024) */

@@ -294,6 +294,17 @@ __device__ __forceinline__ void any_twiddle(float2 (&v)[R], const float2* tw, in
   }
 }
 
+// Sums of squares of values v + shift (x) and v (y), in one order wherever the
+// energies of an image are taken.
+__device__ __forceinline__ float2 add_squares(float2 s, float v, float shift) {
+  const float w = v + shift;
+  return make_float2(fmaf(w, w, s.x), fmaf(v, v, s.y));
+}
+__device__ __forceinline__ float2 wave_sum(float2 s) {
+  for (int o = 32; o > 0; o >>= 1) s = cadd(s, make_float2(__shfl_xor(s.x, o), __shfl_xor(s.y, o)));
+  return s;
+}
+
 // Exchange accesses of butterfly j: the first pass's stores (values of one
 // butterfly, P slots apart between butterflies) and the second pass's loads.
 // ls: log2 of the lines, 0 for a line per row of LDS.

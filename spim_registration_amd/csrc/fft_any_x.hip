@@ -40,6 +40,7 @@ struct XAnyFwdParams {
   AnyFft f;
   int pitch, rows, slots;
   float fill;  // constant gathers: the value outside the source
+  const float2* center;  // (nullable) y: subtracted from the samples of the source
 };
 
 // Second pass of the workgroup's rows after the first pass's exchange, natural
@@ -142,7 +143,7 @@ __device__ __forceinline__ void x_any_forward_body(const XAnyFwdParams& P, int b
       const auto srow = gmem(P.src) + (in ? (int64_t)g.src.x * (gy + (int64_t)g.src.y * gz) : 0);
       const int sx = MODE == kXWrap ? g.src.x / 2 : g.off.x, last = g.src.x - 1;
       const int nx = live ? g.win.x : 0;
-      const float fill = MODE == kXConst ? P.fill : 0.f;
+      const float fill = MODE == kXConst ? P.fill : 0.f, shift = P.center ? gmem(P.center)->y : 0.f;
       auto sample = [&](int x) -> float {
         int gx = sx + x;
         if (MODE == kXWrap) gx = gx >= g.q.x ? gx - g.q.x : gx;
@@ -155,7 +156,7 @@ __device__ __forceinline__ void x_any_forward_body(const XAnyFwdParams& P, int b
         const bool keep = x < nx && (MODE == kXMirror || MODE == kXMirrorAny || (in && at == gx));
         // (bit masks: a conditional use would let the compiler move the load into a branch)
         const unsigned v = __float_as_uint(srow[at]) & (keep ? ~0u : 0u);
-        return __uint_as_float(v | (x < nx && !keep ? __float_as_uint(fill) : 0u));
+        return __uint_as_float(v | (x < nx && !keep ? __float_as_uint(fill) : 0u)) - (keep ? shift : 0.f);
       };
       with_radix_a<RC>(f.a, [&](auto rc) {
         constexpr int R = decltype(rc)::value;
@@ -251,6 +252,12 @@ __device__ __forceinline__ void x_any_inverse_body(const XAnyInvParams& P, int b
   double my_sum = 0.0, my_rsum = 0.0;
   float my_max = -1.f;
   const bool r_rows = EPI != kEpiStore && e.rspec != nullptr;
+  // (less = 0 and shift = 0 change no bit of any value they are subtracted from)
+  float less = 0.f, shift = 0.f;
+  if ((EPI == kEpiQuotient || EPI == kEpiUpdate) && e.center) {
+    less = -gmem(e.center)->x;
+    shift = gmem(e.center)->y;
+  }
   // A wave takes whole rows in pieces of 64 voxels; the inputs of four pieces
   // are loaded before the first is computed (piece by piece, the memory
   // latency of each would follow on the one before).
@@ -295,8 +302,8 @@ __device__ __forceinline__ void x_any_inverse_body(const XAnyInvParams& P, int b
       if (EPI == kEpiStore) {
         *dst = val;
       } else if (EPI == kEpiQuotient) {
-        const float ratio = rl_quotient(val, in0[u]);
-        if (r_rows) fbuf[vofs[u]] = ratio;
+        const float ratio = rl_quotient(val - less, in0[u]);
+        if (r_rows) fbuf[vofs[u]] = ratio - shift;
         else *dst = ratio;
       } else if (EPI == kEpiResidual) {
         float rv = 0.f;
@@ -313,10 +320,10 @@ __device__ __forceinline__ void x_any_inverse_body(const XAnyInvParams& P, int b
       } else {
         float w = in1[u];
         if (e.weight_mode == kWeightVirtual) w = (float)java_min(1.0, (double)w / (double)in2[u] * e.osem);
-        const float next = rl_next_value(in0[u], val, w, e.lambda, inv_lambda);
+        const float next = rl_next_value(in0[u], val - less, w, e.lambda, inv_lambda);
         if (e.keep) gmem(e.keep)[base[u]] = in0[u];
         *dst = next;
-        if (r_rows) fbuf[vofs[u]] = next;
+        if (r_rows) fbuf[vofs[u]] = next - shift;
         const float change = fabsf(next - in0[u]);
         my_sum += (double)change;
         my_max = java_maxf(my_max, change);
@@ -332,7 +339,7 @@ __device__ __forceinline__ void x_any_inverse_body(const XAnyInvParams& P, int b
       for (int h = lane; h < 2 * M - nx; h += 64) {  // the row's positions outside the image
         const int x = h < g.eff_local.x ? h : h + nx, p = x - g.eff_local.x;
         float v = 0.f;
-        if (EPI == kEpiQuotient && x < g.win.x) v = 1.f;
+        if (EPI == kEpiQuotient && x < g.win.x) v = 1.f - shift;
         if (EPI == kEpiUpdate && x < g.win.x) v = wrow[g.eff_local.x + mirror_single(p, nx)];
         wrow[x] = v;
       }
@@ -375,16 +382,17 @@ __device__ __forceinline__ void x_any_inverse_body(const XAnyInvParams& P, int b
       for (int p = wave; p < pieces; p += nw) {
         const int x = p * kEnergyPiece + lane;
         const float* q = fbuf + g.eff_local.x + (x < nx ? x : 0);
-        float s = 0.f;
+        float2 s = make_float2(0.f, 0.f);
         for (int r = 0; r < live_rows; r += 4) {
           float v[4];
 #pragma unroll
           for (int u = 0; u < 4; ++u) v[u] = q[2 * min(r + u, live_rows - 1) * P.slots];
 #pragma unroll
-          for (int u = 0; u < 4; ++u) s += r + u < live_rows ? v[u] * v[u] : 0.f;
+          for (int u = 0; u < 4; ++u)
+            if (r + u < live_rows) s = add_squares(s, v[u], shift);
         }
-        if (x >= nx) s = 0.f;
-        for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
+        if (x >= nx) s = make_float2(0.f, 0.f);
+        s = wave_sum(s);
         if (lane == 0) gmem(e.part_sq)[(int64_t)bx * pieces + p] = s;
       }
     }
@@ -428,10 +436,10 @@ __global__ __launch_bounds__(256) void k_x_any_inverse(XAnyInvParams P, const XA
 int x_any_rows_per_wg(const FftPlan& p) { return row_group_of(p).rows; }
 
 static XAnyFwdParams x_any_fwd_params(const ShapePlan& sp, const ConvGeom& g, const float* src, int gather,
-                                      float2* spec) {
+                                      float2* spec, const float2* center = nullptr) {
   const RowGroup r = row_group_of(sp.px);
   return XAnyFwdParams{g, src, spec, sp.tw_x, any_fft(sp.px), sp.pitch, r.rows, r.slots,
-                       gather == kGatherOne ? 1.f : 0.f};
+                       gather == kGatherOne ? 1.f : 0.f, center};
 }
 
 static hipError_t enqueue_x_forward(int rc, int mode, dim3 grid, dim3 block, size_t lds, hipStream_t stream,
@@ -452,11 +460,11 @@ static hipError_t enqueue_x_forward(int rc, int mode, dim3 grid, dim3 block, siz
 }
 
 hipError_t launch_x_forward_any(const ShapePlan& sp, const ConvGeom& g, const float* src, int gather, float2* spec,
-                                hipStream_t stream) {
+                                hipStream_t stream, const float2* center) {
   const RowGroup r = row_group_of(sp.px);
   const int nrows = g.q.y * g.q.z;
   return enqueue_x_forward(any_class(sp.px), x_gather_of(g, gather), dim3((nrows + r.rows - 1) / r.rows), dim3(r.nt), r.lds, stream,
-                           x_any_fwd_params(sp, g, src, gather, spec), nullptr, nullptr, nullptr, 0);
+                           x_any_fwd_params(sp, g, src, gather, spec, center), nullptr, nullptr, nullptr, 0);
 }
 
 static hipError_t enqueue_x_inverse(int rc, int epi, dim3 grid, dim3 block, size_t lds, hipStream_t stream,

@@ -379,66 +379,116 @@ hipError_t launch_rows(int kind, int cls, const void* items, const int* prefix, 
 // ---------------------------------------------------------------------------
 // energies of what an iteration transforms
 
-__global__ __launch_bounds__(256) void k_rows_energy(const float* img, int nx, int nrows, int per, float* part) {
+__global__ __launch_bounds__(256) void k_rows_energy(const float* img, int nx, int nrows, int per,
+                                                     const float2* center, float2* part) {
   const int row0 = blockIdx.x * per, rows = min(per, nrows - row0), pieces = energy_pieces(nx);
   const int lane = threadIdx.x & 63;
+  const float shift = center ? gmem(center)->y : 0.f;
   for (int p = threadIdx.x >> 6; p < pieces; p += 4) {
     const int x = p * kEnergyPiece + lane;
     const auto src = gmem(img) + (int64_t)row0 * nx + x;
-    float s = 0.f;
+    float2 s = make_float2(0.f, 0.f);
     if (x < nx)
-      for (int r = 0; r < rows; ++r) {
-        const float v = src[(int64_t)r * nx];
-        s += v * v;
-      }
-    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
+      for (int r = 0; r < rows; ++r) s = add_squares(s, src[(int64_t)r * nx] - shift, shift);
+    s = wave_sum(s);
     if (lane == 0) gmem(part)[(int64_t)blockIdx.x * pieces + p] = s;
   }
 }
 
 constexpr int kEnergyThreads = 256;
 
-// A workgroup per slice of a convolution's partials, four loads in flight per
-// thread.
-__global__ __launch_bounds__(kEnergyThreads) void k_energy_sums(const EnergyItem* items) {
-  __shared__ double rs[kEnergyThreads];
-  const EnergyItem E = items[blockIdx.z];
-  const int slice = blockIdx.x, conv = blockIdx.y;
-  if (conv >= E.convs) return;  // uniform
-  const int n = E.nwg * E.pieces;
-  const int lo = (int)((int64_t)n * slice / kEnergySlices), hi = (int)((int64_t)n * (slice + 1) / kEnergySlices);
-  const auto part = gmem(E.part) + (int64_t)conv * n;
-  double s = 0.0;
-#pragma unroll 4
-  for (int i = lo + threadIdx.x; i < hi; i += kEnergyThreads) s += (double)part[i];
-  rs[threadIdx.x] = s;
-  __syncthreads();
-  for (int o = kEnergyThreads / 2; o > 0; o >>= 1) {
-    if (threadIdx.x < o) rs[threadIdx.x] += rs[threadIdx.x + o];
+// Sums of a workgroup's threads, valid in all of them.
+template <int N>
+__device__ __forceinline__ void block_sums(double (&v)[N], double* lds) {
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
     __syncthreads();
+    lds[threadIdx.x] = v[i];
+    __syncthreads();
+    for (int o = kEnergyThreads / 2; o > 0; o >>= 1) {
+      if (threadIdx.x < o) lds[threadIdx.x] += lds[threadIdx.x + o];
+      __syncthreads();
+    }
+    v[i] = lds[0];
   }
-  if (threadIdx.x == 0) gmem(E.sums)[conv * kEnergySlices + slice] = rs[0];
+}
+
+// A workgroup per convolution, region and slice of the region's planes.  A
+// cell (one piece of one workgroup's rows) counts towards every region that it
+// overlaps, and its energy as transformed towards the one that holds its first
+// voxel.
+__global__ __launch_bounds__(kEnergyThreads) void k_energy_sums(const EnergyItem* items) {
+  __shared__ double lds[kEnergyThreads];
+  const EnergyItem E = items[blockIdx.z];
+  const int conv = blockIdx.y, at = blockIdx.x;
+  if (conv >= E.convs || at >= E.regions * E.slices) return;  // uniform
+  const int region = at / E.slices, slice = at - region * E.slices;
+  const auto box = gmem(E.boxes) + region * 6;
+  const int x0 = box[0], x1 = box[1], y0 = box[2], y1 = box[3], z0 = box[4], z1 = box[5];
+  // workgroups that hold a row of planes [z0, z1), and pieces with a voxel of [x0, x1)
+  const int w0 = (int)((int64_t)z0 * E.ny / E.per), w1 = (int)(((int64_t)z1 * E.ny - 1) / E.per) + 1;
+  const int p0 = x0 / kEnergyPiece, np = (x1 - 1) / kEnergyPiece + 1 - p0;
+  const int lo = w0 + (int)((int64_t)(w1 - w0) * slice / E.slices);
+  const int hi = w0 + (int)((int64_t)(w1 - w0) * (slice + 1) / E.slices);
+  const auto part = gmem(E.part) + (int64_t)conv * E.nwg * E.pieces;
+  double v[3] = {0.0, 0.0, 0.0};
+#pragma unroll 2
+  for (int i = threadIdx.x; i < (hi - lo) * np; i += kEnergyThreads) {
+    const int w = lo + i / np, p = p0 + i % np;
+    const float2 s = part[(int64_t)w * E.pieces + p];
+    const int r0 = w * E.per, r1 = min(r0 + E.per, E.nrows) - 1;
+    const int za = r0 / E.ny, ya = r0 - za * E.ny, zb = r1 / E.ny, yb = r1 - zb * E.ny;
+    const bool in_a = za >= z0 && za < z1, in_b = zb >= z0 && zb < z1;
+    const bool over = za == zb       ? in_a && ya < y1 && yb >= y0
+                      : zb == za + 1 ? (in_a && ya < y1) || (in_b && yb >= y0)
+                                     : za < z1 && zb >= z0;
+    if (over) {
+      v[0] += (double)s.x;
+      v[1] += (double)((r1 - r0 + 1) * min(kEnergyPiece, E.nx - p * kEnergyPiece));
+    }
+    if (in_a && ya >= y0 && ya < y1 && p * kEnergyPiece >= x0) v[2] += (double)s.y;
+  }
+  block_sums(v, lds);
+  if (threadIdx.x < 3)
+    gmem(E.sums)[((int64_t)conv * E.regions * E.slices + at) * 3 + threadIdx.x] = v[threadIdx.x];
 }
 
 __global__ __launch_bounds__(kEnergyThreads) void k_energy_check(const EnergyItem* items) {
+  __shared__ double lds[kEnergyThreads];
   const EnergyItem E = items[blockIdx.x];
   int refuse = 0;
-  for (int i = threadIdx.x; i < E.convs * kEnergySlices; i += kEnergyThreads)
-    if (!(gmem(E.sums)[i] < INFINITY)) refuse = 1;  // (squares past the largest float too)
+  for (int c = 0; c < E.convs; ++c) {
+    const auto sums = gmem(E.sums) + (int64_t)c * E.regions * E.slices * 3;
+    double all[1] = {0.0};
+    for (int i = threadIdx.x; i < E.regions * E.slices; i += kEnergyThreads) all[0] += sums[3 * i + 2];
+    block_sums(all, lds);
+    if (!(all[0] < INFINITY)) refuse = 1;  // (also where squares pass the largest float)
+    const double mean = all[0] / ((double)E.nx * E.nrows);
+    for (int r = threadIdx.x; E.limit > 0.0 && r < E.regions; r += kEnergyThreads) {
+      double sq = 0.0, n = 0.0;
+      for (int i = r * E.slices; i < (r + 1) * E.slices; ++i) {
+        sq += sums[3 * i];
+        n += sums[3 * i + 1];
+      }
+      if (!(mean * n <= E.limit * sq)) refuse = 1;
+    }
+  }
   refuse = __syncthreads_or(refuse);
   if (threadIdx.x == 0) *gmem(E.refuse) = refuse;
 }
 
-hipError_t launch_rows_energy(const float* img, Int3 n, int per, float* part, hipStream_t stream) {
+hipError_t launch_rows_energy(const float* img, Int3 n, int per, const float2* center, float2* part,
+                              hipStream_t stream) {
   const int nrows = n.y * n.z;
   (void)hipGetLastError();
-  hipLaunchKernelGGL(k_rows_energy, dim3((nrows + per - 1) / per), dim3(256), 0, stream, img, n.x, nrows, per, part);
+  hipLaunchKernelGGL(k_rows_energy, dim3((nrows + per - 1) / per), dim3(256), 0, stream, img, n.x, nrows, per, center,
+                     part);
   return hipGetLastError();
 }
 
-hipError_t launch_energy_check(const EnergyItem* items, int nitems, int max_convs, hipStream_t stream) {
+hipError_t launch_energy_check(const EnergyItem* items, int nitems, int max_convs, int max_sums, hipStream_t stream) {
   (void)hipGetLastError();
-  hipLaunchKernelGGL(k_energy_sums, dim3(kEnergySlices, max_convs, nitems), dim3(kEnergyThreads), 0, stream, items);
+  hipLaunchKernelGGL(k_energy_sums, dim3(max_sums, max_convs, nitems), dim3(kEnergyThreads), 0, stream, items);
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL(k_energy_check, dim3(nitems), dim3(kEnergyThreads), 0, stream, items);

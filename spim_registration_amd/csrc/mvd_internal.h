@@ -230,10 +230,13 @@ struct EpilogueArgs {
   float2* rspec = nullptr;
   int rpitch = 0;
   double* part_rsum = nullptr;
+  // kEpiQuotient and kEpiUpdate with rspec (nullable): {value added to what the
+  // transform returned, value subtracted from what goes on to the next one}
+  const float2* center = nullptr;
   // kEpiQuotient and kEpiUpdate with rspec (nullable): per workgroup and piece
-  // of kEnergyPiece voxels along x, the sum over its rows of the squares of what
-  // goes on to the transform
-  float* part_sq = nullptr;
+  // of kEnergyPiece voxels along x, the sums over its rows of the squares of the
+  // result and of what goes on to the transform
+  float2* part_sq = nullptr;
   // kEpiUpdate with rspec (nullable): the estimate before the update is kept here
   float* keep = nullptr;
 };
@@ -326,8 +329,9 @@ hipError_t launch_z_any(const ShapePlan& sp, float2* spec, const float2* kspec, 
 hipError_t launch_z_any_grad(const ShapePlan& sp, float2* spec, const float2* what, const float2* khat, float2* corr,
                              int mode, int first, Int3 shift, int zlo, int zhi, int kz, const double* rsum,
                              float2* adj, bool adj_add, hipStream_t stream);
+// center (nullable): center->y is subtracted from the samples of the source.
 hipError_t launch_x_forward_any(const ShapePlan& sp, const ConvGeom& g, const float* src, int gather, float2* spec,
-                                hipStream_t stream);
+                                hipStream_t stream, const float2* center = nullptr);
 hipError_t launch_x_inverse_any(const ShapePlan& sp, const ConvGeom& g, const float2* spec, const EpilogueArgs& e,
                                 hipStream_t stream, int nwg);
 
@@ -403,18 +407,21 @@ hipError_t launch_to_slabs(const ShapePlan& sp, const float2* in, float2* out, h
 int build_rows_params(const RowsPass& d, void* out, int* gx, int* gy, int* cls, int* threads, size_t* lds);
 hipError_t launch_rows(int kind, int cls, const void* items, const int* prefix, const int* gx, int nitems, int nwg,
                        int threads, size_t lds, hipStream_t stream);
-// What the convolutions of one iteration by rows transform: the partials of
-// their energies (EpilogueArgs::part_sq, one set per convolution).
-constexpr int kEnergySlices = 32;
+// The check of one iteration by rows: the partials of its convolutions'
+// energies (EpilogueArgs::part_sq), summed over regions of the image.
 struct EnergyItem {
-  const float* part;  // [convs][nwg][pieces]
-  double* sums;       // [convs][kEnergySlices]
-  int* refuse;        // set to 1 if one of them holds a NaN or an infinity, else to 0
-  int convs, nwg, pieces;
+  const float2* part;  // [convs][nwg][pieces]
+  const int* boxes;    // [regions][6], x0, x1, y0, y1, z0, z1: they partition the image
+  double* sums;        // [convs][regions * slices][3]
+  int* refuse;         // the verdict, 1 or 0
+  int convs, regions, slices, nwg, pieces, per;  // per: rows a workgroup
+  int nx, ny, nrows;
+  double limit;  // of the image's mean square as transformed over a region's mean square; 0: any finite one
 };
-// The partials of an image, `per` rows a workgroup.
-hipError_t launch_rows_energy(const float* img, Int3 n, int per, float* part, hipStream_t stream);
-hipError_t launch_energy_check(const EnergyItem* items, int nitems, int max_convs, hipStream_t stream);
+// The partials of an image less center->y (nullable), `per` rows a workgroup.
+hipError_t launch_rows_energy(const float* img, Int3 n, int per, const float2* center, float2* part,
+                              hipStream_t stream);
+hipError_t launch_energy_check(const EnergyItem* items, int nitems, int max_convs, int max_sums, hipStream_t stream);
 constexpr int kMaxParamBytes = 640;
 bool pass_is_fast(const PassDesc& d);
 bool pass_is_any(const PassDesc& d);

@@ -415,7 +415,7 @@ struct PassLaunch {
   bool lines = false;  // z pass with one kernel spectrum for all items: grid (lx, ly) of lines
   int lx = 0, ly = 0;
   bool reduce = false;
-  bool energy = false;  // check of the energies of an iteration by rows; lx: convolutions of an item at most
+  bool energy = false;  // check of the energies of an iteration by rows; lx, ly: convolutions and sums of an item at most
   size_t lds = 0;
   const LaunchTables* tab = nullptr;  // uploaded before the launch
   size_t items_at = 0, prefix_at = 0, gx_at = 0;
@@ -762,15 +762,27 @@ struct mvd_session {
   //
   // One value that is no finite number reaches every value of its rows, then of
   // its tile: in block windows it reaches its blocks, in one window the image.
-  // Where those differ (`guard`), every iteration sums the squares of what its
-  // convolutions transform, and one that met a NaN or an infinity is taken back
+  // And the rounding of an FP32 transform follows the root mean square of all
+  // that it transforms, in block windows of a block: by rows a bright part of the
+  // image costs the dim blocks their precision.  Where those differ (`guard`),
+  // every iteration sums the squares of what its convolutions transform, and one
+  // that met a NaN, an infinity or a block too dim (kEnergyLimit) is taken back
   // and repeated, and the later ones run, in block windows (use_windows).  The
   // ratio image, which iterations by rows leave alone, holds the estimate
   // meanwhile.
+  //
+  // Sessions of several blocks transform the estimate less the views' mean and
+  // the ratio less one (`centred`; a constant's convolution is that constant
+  // times the kernel's sum), which leaves less to round: see kEnergyLimit.
   struct RowConv {
-    bool guard = false;
+    bool guard = false, centred = false;  // (only together with `on`)
     DeviceBuf energy;  // partials of the squares per convolution, estimate of view 0 first
     DeviceBuf esums;   // their sums (double), then the check's verdict (int)
+    DeviceBuf boxes;   // the blocks (EnergyItem)
+    int regions = 1, slices = 1;
+    float mean = 0.f;  // of the views
+    std::vector<float2> center_host;  // per view and convolution (EpilogueArgs::center)
+    DeviceBuf centers;
     bool on = false, shared = false, consts = false;  // shared: the views' own spectra have this shape
     const ShapePlan* plan = nullptr;
     Int3 kd{0, 0, 0}, win{0, 0, 0};
@@ -983,7 +995,7 @@ int build_rows_launches(const std::vector<RowsPass>& passes, LaunchTables* tab, 
 
 hipError_t enqueue_pass_launch(const PassLaunch& L, hipStream_t st) {
   if (L.reduce) return launch_reduce_stats_batch(static_cast<const ReduceItem*>(L.items()), L.nitems, st);
-  if (L.energy) return launch_energy_check(static_cast<const EnergyItem*>(L.items()), L.nitems, L.lx, st);
+  if (L.energy) return launch_energy_check(static_cast<const EnergyItem*>(L.items()), L.nitems, L.lx, L.ly, st);
   if (L.lines) return launch_z_lines(L.cls, L.items(), L.nitems, L.lx, L.ly, st, L.table);
   if (L.path == 2)
     return launch_batch_xy(L.kind, L.cls, L.items(), L.prefix(), L.gx(), L.nitems, L.nwg, st,
@@ -1103,11 +1115,24 @@ int rows_length(int w, int most, bool columns, double* cost) {
   return best;
 }
 
+// How many times the mean square that the rows transform (centred) may be that
+// of a block's own values: at most so many that no block is further from 64 bits
+// than in its windows.  Errors by rows over errors in windows, worst block of
+// 421x337x203, 512x512x256 and 300x333x150 after 5 or 6 iterations, rms and
+// maximum, by the largest such ratio met: 0.09 to 0.13 (beads on a background of
+// 100) 0.70 and 0.75; 0.16 to 0.23 (one half 1.4 times brighter) 0.74 and 0.68;
+// 0.41 to 0.61 (one half twice as bright, or a background of 20) 0.91 and 0.91;
+// 0.97 (a background of 5) 1.15 and 1.54; 2.7 to 3.2 (one half four times
+// brighter) 1.33 and 1.15.  Uncentred: 1.28 and 1.37 on the first of these data.
+constexpr double kEnergyLimit = 0.6;
+
+int first_iteration_sums(mvd_session* s, float* counts, double* sum, unsigned long long* cnt);
+
 // No iteration by rows until the next mvd_prepare; its buffers go.
 void drop_rows(mvd_session* s) {
   auto& r = s->rc;
-  r.on = r.consts = r.guard = false;
-  for (DeviceBuf* b : {&r.rows, &r.planes, &r.plain, &r.energy, &r.esums}) *b = DeviceBuf();
+  r.on = r.consts = r.guard = r.centred = false;
+  for (DeviceBuf* b : {&r.rows, &r.planes, &r.plain, &r.energy, &r.esums, &r.boxes, &r.centers}) *b = DeviceBuf();
   for (auto& v : s->views) {
     v.r1hat = DeviceBuf();
     v.r2hat = DeviceBuf();
@@ -1122,7 +1147,7 @@ void drop_rows(mvd_session* s) {
 // is about as cheap (within 10 %), so that the gradient uses the same spectra.
 int plan_rows(mvd_session* s) {
   auto& r = s->rc;
-  r.on = r.consts = r.guard = false;
+  r.on = r.consts = r.guard = r.centred = false;
   if (s->windows_only) return 0;
   const Int3 n = s->img, kd = s->views[0].kd;
   for (auto& v : s->views)
@@ -1185,7 +1210,33 @@ int plan_rows(mvd_session* s) {
   r.geom = g;
   const int per = x_any_rows_per_wg(r.plan->px);
   r.nwg = (n.y * n.z + per - 1) / per;
-  r.guard = v0.blocks.size() > 1 || r.tiles.size() > 1;
+  // blocks that the check's cells cannot tell apart stay in their windows
+  const bool split = v0.blocks.size() > 1;
+  if (split && (v0.blocks[0].eff_size.x < kEnergyPiece || v0.blocks[0].eff_size.y < per || v0.blocks.size() > 4096))
+    return 0;
+  if (split) {
+    double sum = 0;
+    unsigned long long cnt = 0;
+    if (int rc = first_iteration_sums(s, nullptr, &sum, &cnt)) return rc;
+    r.mean = cnt > 0 && std::isfinite(sum) ? (float)(sum / (double)cnt) : 0.f;
+  }
+  if (split || r.tiles.size() > 1) {
+    std::vector<int> boxes = {0, n.x, 0, n.y, 0, n.z};
+    if (split) {
+      boxes.clear();
+      for (auto& b : v0.blocks)
+        for (auto at : {std::make_pair(b.eff_offset.x, b.eff_size.x), std::make_pair(b.eff_offset.y, b.eff_size.y),
+                        std::make_pair(b.eff_offset.z, b.eff_size.z)})
+          boxes.insert(boxes.end(), {at.first, at.first + at.second});
+    }
+    r.regions = (int)boxes.size() / 6;
+    r.slices = std::max(1, std::min(32, 64 / r.regions));
+    MVD_CHECK(r.boxes.ensure(sizeof(int) * boxes.size()));
+    MVD_CHECK(hipMemcpy(r.boxes.p, boxes.data(), sizeof(int) * boxes.size(), hipMemcpyHostToDevice));
+    MVD_CHECK(r.centers.ensure(sizeof(float2) * 2 * s->nviews));
+  }
+  r.guard = split || r.tiles.size() > 1;
+  r.centred = split;
   r.on = true;
   if (r.shared) return 0;
   // the kernels' spectra now, the rest at the first iteration (reserve_rows)
@@ -1201,9 +1252,35 @@ int plan_rows(mvd_session* s) {
 
 // Where the partials of convolution `conv` (0 .. 2 nviews - 1, two of a view in
 // the order of an iteration) are.
-float* energy_of(mvd_session* s, int conv) {
+float2* energy_of(mvd_session* s, int conv) {
   const size_t n = (size_t)s->rc.nwg * energy_pieces(s->img.x);
-  return s->rc.energy.as<float>() + n * conv;
+  return s->rc.energy.as<float2>() + n * conv;
+}
+
+// Whether the session's iterations are checked.
+bool guarded(const mvd_session* s) { return s->rc.on && s->rc.guard; }
+
+const float2* center_of(mvd_session* s, int v, int conv) {
+  return s->rc.centred ? s->rc.centers.as<float2>() + 2 * v + conv : nullptr;
+}
+
+// {mean times kernel1's sum, one} and {kernel2's sum, mean} of every view.
+int upload_centers(mvd_session* s) {
+  auto& r = s->rc;
+  if (!r.on || !r.centred) return 0;
+  auto sum = [](const std::vector<float>& k) {
+    double t = 0;
+    for (float x : k) t += x;
+    return t;
+  };
+  r.center_host.clear();
+  for (auto& v : s->views) {
+    r.center_host.push_back(make_float2((float)(r.mean * sum(v.k1)), 1.f));
+    r.center_host.push_back(make_float2((float)sum(v.k2), r.mean));
+  }
+  MVD_CHECK(hipMemcpyAsync(r.centers.p, r.center_host.data(), sizeof(float2) * r.center_host.size(),
+                           hipMemcpyHostToDevice, s->stream));
+  return 0;
 }
 
 int add_energy_check(const std::vector<EnergyItem>& items, LaunchTables* tab, std::vector<PassLaunch>* out) {
@@ -1212,7 +1289,10 @@ int add_energy_check(const std::vector<EnergyItem>& items, LaunchTables* tab, st
   L.energy = true;
   L.timing = kTReduce;
   L.nitems = (int)items.size();
-  for (auto& i : items) L.lx = std::max(L.lx, i.convs);
+  for (auto& i : items) {
+    L.lx = std::max(L.lx, i.convs);
+    L.ly = std::max(L.ly, i.regions * i.slices);
+  }
   L.tab = tab;
   L.items_at = tab->add(items.data(), sizeof(EnergyItem) * items.size());
   out->push_back(std::move(L));
@@ -1223,8 +1303,23 @@ int add_energy_check(const std::vector<EnergyItem>& items, LaunchTables* tab, st
 EnergyItem energy_item(mvd_session* s, int* refuse) {
   auto& r = s->rc;
   const int convs = 2 * s->nviews;
-  if (!refuse) refuse = reinterpret_cast<int*>(r.esums.as<double>() + convs * kEnergySlices);
-  return {r.energy.as<float>(), r.esums.as<double>(), refuse, convs, r.nwg, energy_pieces(s->img.x)};
+  if (!refuse) refuse = reinterpret_cast<int*>(r.esums.as<double>() + 3 * (size_t)convs * r.regions * r.slices);
+  EnergyItem e{};
+  e.part = r.energy.as<float2>();
+  e.boxes = r.boxes.as<int>();
+  e.sums = r.esums.as<double>();
+  e.refuse = refuse;
+  e.convs = convs;
+  e.regions = r.regions;
+  e.slices = r.slices;
+  e.nwg = r.nwg;
+  e.pieces = energy_pieces(s->img.x);
+  e.per = x_any_rows_per_wg(r.plan->px);
+  e.nx = s->img.x;
+  e.ny = s->img.y;
+  e.nrows = s->img.y * s->img.z;
+  e.limit = r.centred ? kEnergyLimit : 0.0;
+  return e;
 }
 
 // The y and z passes and the x pass of one convolution of view v by rows.
@@ -1271,6 +1366,7 @@ void rows_pass_descs(mvd_session* s, int v, int conv, std::vector<RowsPass> (&pa
   x.e.rspec = r.rows.as<float2>();
   x.e.rpitch = r.plan->pitch;
   // the ratio goes to the view's second convolution, the estimate to the next view's first
+  x.e.center = center_of(s, v, conv);
   if (r.guard) x.e.part_sq = energy_of(s, conv == 0 ? 2 * v + 1 : 2 * ((v + 1) % s->nviews));
   if (r.guard && conv == 1 && v == 0) x.e.keep = s->d_ratio.as<float>();
   xinv->push_back(x);
@@ -1287,8 +1383,8 @@ bool reserve_rows(mvd_session* s) {
   const std::pair<DeviceBuf*, size_t> sizes[] = {
       {&r.rows, sizeof(float2) * r.plan->pitch * (nrows + 1)},
       {&r.planes, sizeof(float2) * (slab_elems(*r.plan, n.z) * r.tiles.size() + slab_elems(*r.plan, 1))},
-      {&r.energy, sizeof(float) * convs * r.nwg * energy_pieces(n.x)},
-      {&r.esums, r.guard ? sizeof(double) * (convs * kEnergySlices + 1) : 0}};
+      {&r.energy, sizeof(float2) * convs * r.nwg * energy_pieces(n.x)},
+      {&r.esums, r.guard ? sizeof(double) * (3 * convs * r.regions * r.slices + 1) : 0}};
   for (auto& b : sizes)
     if (b.first->ensure(b.second) != hipSuccess) {
       (void)hipGetLastError();
@@ -1297,8 +1393,8 @@ bool reserve_rows(mvd_session* s) {
   return true;
 }
 
-// The spectra of the constant one that the ratio has outside the image: a row
-// along x, a plane along x and y.  After reserve_rows.
+// The spectra of the constant one that the ratio has outside the image (zero
+// where it is centred): a row along x, a plane along x and y.  After reserve_rows.
 int ensure_rows(mvd_session* s) {
   auto& r = s->rc;
   if (r.consts) return 0;
@@ -1310,7 +1406,8 @@ int ensure_rows(mvd_session* s) {
   g.off = {0, 1, 1};  // outside the source: the constant everywhere
   g.win = {r.win.x, 1, 1};
   g.q = {q.x, 1, 1};
-  MVD_CHECK(launch_x_forward_any(*r.plan, g, s->d_psi.as<float>(), kGatherOne, crow, s->stream));
+  MVD_CHECK(launch_x_forward_any(*r.plan, g, s->d_psi.as<float>(), r.centred ? kGatherZero : kGatherOne, crow,
+                                 s->stream));
   RowsPass y{};
   y.kind = kPassYForward;
   y.sp = r.plan;
@@ -1336,10 +1433,12 @@ hipError_t rows_start(mvd_session* s, hipStream_t st) {
   auto& r = s->rc;
   if (r.guard) {
     const hipError_t e =
-        launch_rows_energy(s->d_psi.as<float>(), s->img, x_any_rows_per_wg(r.plan->px), energy_of(s, 0), st);
+        launch_rows_energy(s->d_psi.as<float>(), s->img, x_any_rows_per_wg(r.plan->px), center_of(s, 0, 1),
+                           energy_of(s, 0), st);
     if (e != hipSuccess) return e;
   }
-  return launch_x_forward_any(*r.plan, r.geom, s->d_psi.as<float>(), kGatherMirror, r.rows.as<float2>(), st);
+  return launch_x_forward_any(*r.plan, r.geom, s->d_psi.as<float>(), kGatherMirror, r.rows.as<float2>(), st,
+                              center_of(s, 0, 1));
 }
 
 // The estimate before the iteration by rows, which its first update has kept.
@@ -1372,7 +1471,7 @@ int build_block_batch(mvd_session* s) {
           if ((rc = build_rows_launches(p, &bb.tables, &bb.view[v]))) return rc;
         if ((rc = build_pass_launches(xinv, &bb.tables, &bb.view[v]))) return rc;
         // (before the last update makes the estimate of the next iteration)
-        if (s->rc.guard && conv == 0 && v == s->nviews - 1)
+        if (guarded(s) && conv == 0 && v == s->nviews - 1)
           if ((rc = add_energy_check({energy_item(s, nullptr)}, &bb.tables, &bb.view[v]))) return rc;
       }
     MVD_CHECK(bb.tables.upload());
@@ -2311,7 +2410,7 @@ int mvd_prepare(mvd_session* s, int psf_type, double lambda, const int* block_xy
     if (rc) return rc;
   }
   int rc = ensure_workspace(s);
-  if (rc) return rc;
+  if (rc || (rc = upload_centers(s))) return rc;
   MVD_CHECK(hipStreamSynchronize(s->stream));
   ++s->epoch;
   s->prepared = true;
@@ -2346,7 +2445,7 @@ int mvd_set_psf(mvd_session* s, int view, const float* psf) {
   if (!s->rc.on) s->bb.built = false;  // (by rows: the launch lists name the same buffers)
   int rc = init_view(s, view);
   if (rc) return rc;
-  if ((rc = view_spectra(s, view))) return rc;
+  if ((rc = view_spectra(s, view)) || (rc = upload_centers(s))) return rc;
   MVD_CHECK(hipStreamSynchronize(s->stream));
   return 0;
 }
@@ -2368,6 +2467,7 @@ int mvd_set_psfs(mvd_session* s, const float* const* psfs) {
     int rc = view_spectra(s, v);
     if (rc) return rc;
   }
+  if (int rc = upload_centers(s)) return rc;
   MVD_CHECK(hipStreamSynchronize(s->stream));
   return 0;
 }
@@ -2429,7 +2529,7 @@ int mvd_iterate(mvd_session* s, int n, double* stats) {
     s->timer.end(s->stream, kTXForward);
   }
   for (int it = 0; it < n; ++it) {
-    const bool guard = s->rc.on && s->rc.guard;
+    const bool guard = guarded(s);
     int rc = enqueue_iteration(s, it);
     if (rc) return rc;
     if (!guard) continue;
@@ -3002,7 +3102,7 @@ int build_batch(mvd_batch* b) {
       if (conv == 0) {
         std::vector<EnergyItem> checks;
         for (size_t si = 0; si < b->stacks.size(); ++si)
-          if (b->stacks[si]->rc.guard && v == b->stacks[si]->nviews - 1)
+          if (guarded(b->stacks[si]) && v == b->stacks[si]->nviews - 1)
             checks.push_back(energy_item(b->stacks[si], b->refuse.as<int>() + si));
         if (int rc = add_energy_check(checks, &b->tables, &b->launches)) return rc;
       }
@@ -3122,7 +3222,7 @@ int mvd_batch_iterate(mvd_batch* b, int n, double* stats) {
     if (s->rc.on) MVD_CHECK(rows_start(s, b->stream));
   for (int it = 0; it < n; ++it) {
     bool guard = false;
-    for (auto* s : b->stacks) guard = guard || s->rc.guard;
+    for (auto* s : b->stacks) guard = guard || guarded(s);
     if (b->use_graph) {
       MVD_CHECK(hipGraphLaunch(b->exec, b->stream));
     } else {
@@ -3138,7 +3238,7 @@ int mvd_batch_iterate(mvd_batch* b, int n, double* stats) {
     MVD_CHECK(hipStreamSynchronize(b->stream));
     bool left = false;
     for (size_t si = 0; si < b->stacks.size(); ++si)
-      if (b->stacks[si]->rc.guard && refuse[si]) {
+      if (guarded(b->stacks[si]) && refuse[si]) {
         left = true;
         int rc = repeat_in_windows(b, si, it);
         if (rc) return rc;
