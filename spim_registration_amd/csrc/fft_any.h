@@ -300,9 +300,26 @@ __device__ __forceinline__ float2 add_squares(float2 s, float v, float shift) {
   const float w = v + shift;
   return make_float2(fmaf(w, w, s.x), fmaf(v, v, s.y));
 }
-__device__ __forceinline__ float2 wave_sum(float2 s) {
-  for (int o = 32; o > 0; o >>= 1) s = cadd(s, make_float2(__shfl_xor(s.x, o), __shfl_xor(s.y, o)));
-  return s;
+// Sum over each half of a wavefront, in lanes 31 and 63 only: within rows of 16
+// lanes by shifts, then from row 0 to 1 and 2 to 3 by a broadcast of the last
+// lane, all in the VALU.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ float add_lanes(float v) {
+  return v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, ROWS, 0xf, false));
+}
+__device__ __forceinline__ float half_wave_sum(float v) {
+  v = add_lanes<0x111, 0xf>(v);  // row_shr:1, 2, 4, 8
+  v = add_lanes<0x112, 0xf>(v);
+  v = add_lanes<0x114, 0xf>(v);
+  v = add_lanes<0x118, 0xf>(v);
+  return add_lanes<0x142, 0xa>(v);  // row_bcast:15 to rows 1 and 3
+}
+// The energy of a half wavefront's pairs of columns x and x + 1 (a, b) within
+// [0, nx), in its last lane.
+__device__ __forceinline__ float2 energy_of_pair(float2 a, float2 b, int x, int nx) {
+  const bool in_a = (unsigned)x < (unsigned)nx, in_b = (unsigned)(x + 1) < (unsigned)nx;
+  const float2 s = make_float2((in_a ? a.x : 0.f) + (in_b ? b.x : 0.f), (in_a ? a.y : 0.f) + (in_b ? b.y : 0.f));
+  return make_float2(half_wave_sum(s.x), half_wave_sum(s.y));
 }
 
 // Exchange accesses of butterfly j: the first pass's stores (values of one

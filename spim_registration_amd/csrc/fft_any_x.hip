@@ -155,8 +155,9 @@ __device__ __forceinline__ void x_any_forward_body(const XAnyFwdParams& P, int b
         const int at = MODE == kXMirrorAny ? gx : min(max(gx, 0), last);
         const bool keep = x < nx && (MODE == kXMirror || MODE == kXMirrorAny || (in && at == gx));
         // (bit masks: a conditional use would let the compiler move the load into a branch)
-        const unsigned v = __float_as_uint(srow[at]) & (keep ? ~0u : 0u);
-        return __uint_as_float(v | (x < nx && !keep ? __float_as_uint(fill) : 0u)) - (keep ? shift : 0.f);
+        const unsigned m = keep ? ~0u : 0u, v = __float_as_uint(srow[at]) & m;
+        return __uint_as_float(v | (x < nx && !keep ? __float_as_uint(fill) : 0u)) -
+               __uint_as_float(__float_as_uint(shift) & m);
       };
       with_radix_a<RC>(f.a, [&](auto rc) {
         constexpr int R = decltype(rc)::value;
@@ -376,24 +377,21 @@ __device__ __forceinline__ void x_any_inverse_body(const XAnyInvParams& P, int b
     const int l = (int)__umulhi((unsigned)threadIdx.x, f.mb), j = threadIdx.x - l * f.b;
     __syncthreads();
     if ((EPI == kEpiQuotient || EPI == kEpiUpdate) && e.part_sq) {
-      // the rows' energies, a wave per piece, from LDS once more (6 views of
-      // 512x512x256: quotient 249 -> 266 us, update 418 -> 431)
-      const int pieces = energy_pieces(nx);
-      for (int p = wave; p < pieces; p += nw) {
-        const int x = p * kEnergyPiece + lane;
-        const float* q = fbuf + g.eff_local.x + (x < nx ? x : 0);
-        float2 s = make_float2(0.f, 0.f);
-        for (int r = 0; r < live_rows; r += 4) {
-          float v[4];
-#pragma unroll
-          for (int u = 0; u < 4; ++u) v[u] = q[2 * min(r + u, live_rows - 1) * P.slots];
-#pragma unroll
-          for (int u = 0; u < 4; ++u)
-            if (r + u < live_rows) s = add_squares(s, v[u], shift);
+      // the rows' energies from LDS, two neighbouring values of every row a
+      // thread, a piece per half wavefront: the quotient of 880x880x440 1459 ->
+      // 1538 us (1614 with single values and shuffles through LDS)
+      const int pieces = energy_pieces(2 * M);
+      for (int c = threadIdx.x; c < pieces * 32; c += blockDim.x) {
+        const float2* q = buf + min(c, M - 1);
+        float2 a = make_float2(0.f, 0.f), b = a;
+#pragma unroll 4
+        for (int r = 0; r < live_rows; ++r) {
+          const float2 v = q[r * P.slots];
+          a = add_squares(a, v.x, shift);
+          b = add_squares(b, v.y, shift);
         }
-        if (x >= nx) s = make_float2(0.f, 0.f);
-        s = wave_sum(s);
-        if (lane == 0) gmem(e.part_sq)[(int64_t)bx * pieces + p] = s;
+        const float2 s = energy_of_pair(a, b, 2 * c - g.eff_local.x, nx);
+        if ((lane & 31) == 31) gmem(e.part_sq)[(int64_t)bx * pieces + (c >> 5)] = s;
       }
     }
     with_radix_a<RC>(f.a, [&](auto rc) {

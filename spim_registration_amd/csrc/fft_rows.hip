@@ -379,19 +379,22 @@ hipError_t launch_rows(int kind, int cls, const void* items, const int* prefix, 
 // ---------------------------------------------------------------------------
 // energies of what an iteration transforms
 
-__global__ __launch_bounds__(256) void k_rows_energy(const float* img, int nx, int nrows, int per,
+__global__ __launch_bounds__(256) void k_rows_energy(const float* img, int nx, int nrows, int ex, int pieces, int per,
                                                      const float2* center, float2* part) {
-  const int row0 = blockIdx.x * per, rows = min(per, nrows - row0), pieces = energy_pieces(nx);
-  const int lane = threadIdx.x & 63;
+  const int row0 = blockIdx.x * per, rows = min(per, nrows - row0);
   const float shift = center ? gmem(center)->y : 0.f;
-  for (int p = threadIdx.x >> 6; p < pieces; p += 4) {
-    const int x = p * kEnergyPiece + lane;
-    const auto src = gmem(img) + (int64_t)row0 * nx + x;
-    float2 s = make_float2(0.f, 0.f);
-    if (x < nx)
-      for (int r = 0; r < rows; ++r) s = add_squares(s, src[(int64_t)r * nx] - shift, shift);
-    s = wave_sum(s);
-    if (lane == 0) gmem(part)[(int64_t)blockIdx.x * pieces + p] = s;
+  for (int c = threadIdx.x; c < pieces * 32; c += 256) {
+    const int x = 2 * c - ex;
+    const auto src = gmem(img) + (int64_t)row0 * nx;
+    const int xa = min(max(x, 0), nx - 1), xb = min(max(x + 1, 0), nx - 1);
+    float2 a = make_float2(0.f, 0.f), b = a;
+#pragma unroll 4
+    for (int r = 0; r < rows; ++r) {
+      a = add_squares(a, src[(int64_t)r * nx + xa] - shift, shift);
+      b = add_squares(b, src[(int64_t)r * nx + xb] - shift, shift);
+    }
+    const float2 s = energy_of_pair(a, b, x, nx);
+    if ((threadIdx.x & 31) == 31) gmem(part)[(int64_t)blockIdx.x * pieces + (c >> 5)] = s;
   }
 }
 
@@ -427,7 +430,7 @@ __global__ __launch_bounds__(kEnergyThreads) void k_energy_sums(const EnergyItem
   const int x0 = box[0], x1 = box[1], y0 = box[2], y1 = box[3], z0 = box[4], z1 = box[5];
   // workgroups that hold a row of planes [z0, z1), and pieces with a voxel of [x0, x1)
   const int w0 = (int)((int64_t)z0 * E.ny / E.per), w1 = (int)(((int64_t)z1 * E.ny - 1) / E.per) + 1;
-  const int p0 = x0 / kEnergyPiece, np = (x1 - 1) / kEnergyPiece + 1 - p0;
+  const int p0 = (x0 + E.ex) / kEnergyPiece, np = (x1 - 1 + E.ex) / kEnergyPiece + 1 - p0;
   const int lo = w0 + (int)((int64_t)(w1 - w0) * slice / E.slices);
   const int hi = w0 + (int)((int64_t)(w1 - w0) * (slice + 1) / E.slices);
   const auto part = gmem(E.part) + (int64_t)conv * E.nwg * E.pieces;
@@ -442,11 +445,12 @@ __global__ __launch_bounds__(kEnergyThreads) void k_energy_sums(const EnergyItem
     const bool over = za == zb       ? in_a && ya < y1 && yb >= y0
                       : zb == za + 1 ? (in_a && ya < y1) || (in_b && yb >= y0)
                                      : za < z1 && zb >= z0;
+    const int xa = max(p * kEnergyPiece - E.ex, 0), xb = min((p + 1) * kEnergyPiece - E.ex, E.nx);
     if (over) {
       v[0] += (double)s.x;
-      v[1] += (double)((r1 - r0 + 1) * min(kEnergyPiece, E.nx - p * kEnergyPiece));
+      v[1] += (double)((r1 - r0 + 1) * (xb - xa));
     }
-    if (in_a && ya >= y0 && ya < y1 && p * kEnergyPiece >= x0) v[2] += (double)s.y;
+    if (in_a && ya >= y0 && ya < y1 && xa >= x0) v[2] += (double)s.y;
   }
   block_sums(v, lds);
   if (threadIdx.x < 3)
@@ -477,12 +481,12 @@ __global__ __launch_bounds__(kEnergyThreads) void k_energy_check(const EnergyIte
   if (threadIdx.x == 0) *gmem(E.refuse) = refuse;
 }
 
-hipError_t launch_rows_energy(const float* img, Int3 n, int per, const float2* center, float2* part,
-                              hipStream_t stream) {
+hipError_t launch_rows_energy(const float* img, Int3 n, int ex, int pieces, int per, const float2* center,
+                              float2* part, hipStream_t stream) {
   const int nrows = n.y * n.z;
   (void)hipGetLastError();
-  hipLaunchKernelGGL(k_rows_energy, dim3((nrows + per - 1) / per), dim3(256), 0, stream, img, n.x, nrows, per, center,
-                     part);
+  hipLaunchKernelGGL(k_rows_energy, dim3((nrows + per - 1) / per), dim3(256), 0, stream, img, n.x, nrows, ex, pieces,
+                     per, center, part);
   return hipGetLastError();
 }
 

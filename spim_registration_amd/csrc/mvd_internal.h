@@ -234,14 +234,14 @@ struct EpilogueArgs {
   // transform returned, value subtracted from what goes on to the next one}
   const float2* center = nullptr;
   // kEpiQuotient and kEpiUpdate with rspec (nullable): per workgroup and piece
-  // of kEnergyPiece voxels along x, the sums over its rows of the squares of the
-  // result and of what goes on to the transform
+  // of kEnergyPiece samples of a window row, the sums over its rows of the squares
+  // of the result and of what goes on to the transform, the image's voxels alone
   float2* part_sq = nullptr;
   // kEpiUpdate with rspec (nullable): the estimate before the update is kept here
   float* keep = nullptr;
 };
 constexpr int kEnergyPiece = 64;
-__host__ __device__ inline int energy_pieces(int nx) { return (nx + kEnergyPiece - 1) / kEnergyPiece; }
+__host__ __device__ inline int energy_pieces(int qx) { return (qx + kEnergyPiece - 1) / kEnergyPiece; }
 
 // Launchers (all asynchronous on `stream`).
 hipError_t launch_x_forward(const ShapePlan& sp, const ConvGeom& g, const float* src, int gather, float2* spec,
@@ -415,12 +415,12 @@ struct EnergyItem {
   double* sums;        // [convs][regions * slices][3]
   int* refuse;         // the verdict, 1 or 0
   int convs, regions, slices, nwg, pieces, per;  // per: rows a workgroup
-  int nx, ny, nrows;
+  int nx, ny, nrows, ex;  // ex: the image's first voxel in a window row
   double limit;  // of the image's mean square as transformed over a region's mean square; 0: any finite one
 };
 // The partials of an image less center->y (nullable), `per` rows a workgroup.
-hipError_t launch_rows_energy(const float* img, Int3 n, int per, const float2* center, float2* part,
-                              hipStream_t stream);
+hipError_t launch_rows_energy(const float* img, Int3 n, int ex, int pieces, int per, const float2* center,
+                              float2* part, hipStream_t stream);
 hipError_t launch_energy_check(const EnergyItem* items, int nitems, int max_convs, int max_sums, hipStream_t stream);
 constexpr int kMaxParamBytes = 640;
 bool pass_is_fast(const PassDesc& d);

@@ -1253,7 +1253,7 @@ int plan_rows(mvd_session* s) {
 // Where the partials of convolution `conv` (0 .. 2 nviews - 1, two of a view in
 // the order of an iteration) are.
 float2* energy_of(mvd_session* s, int conv) {
-  const size_t n = (size_t)s->rc.nwg * energy_pieces(s->img.x);
+  const size_t n = (size_t)s->rc.nwg * energy_pieces(s->rc.plan->q.x);
   return s->rc.energy.as<float2>() + n * conv;
 }
 
@@ -1313,7 +1313,8 @@ EnergyItem energy_item(mvd_session* s, int* refuse) {
   e.regions = r.regions;
   e.slices = r.slices;
   e.nwg = r.nwg;
-  e.pieces = energy_pieces(s->img.x);
+  e.pieces = energy_pieces(r.plan->q.x);
+  e.ex = r.geom.eff_local.x;
   e.per = x_any_rows_per_wg(r.plan->px);
   e.nx = s->img.x;
   e.ny = s->img.y;
@@ -1383,7 +1384,7 @@ bool reserve_rows(mvd_session* s) {
   const std::pair<DeviceBuf*, size_t> sizes[] = {
       {&r.rows, sizeof(float2) * r.plan->pitch * (nrows + 1)},
       {&r.planes, sizeof(float2) * (slab_elems(*r.plan, n.z) * r.tiles.size() + slab_elems(*r.plan, 1))},
-      {&r.energy, sizeof(float2) * convs * r.nwg * energy_pieces(n.x)},
+      {&r.energy, sizeof(float2) * convs * r.nwg * energy_pieces(r.plan->q.x)},
       {&r.esums, r.guard ? sizeof(double) * (3 * convs * r.regions * r.slices + 1) : 0}};
   for (auto& b : sizes)
     if (b.first->ensure(b.second) != hipSuccess) {
@@ -1433,8 +1434,8 @@ hipError_t rows_start(mvd_session* s, hipStream_t st) {
   auto& r = s->rc;
   if (r.guard) {
     const hipError_t e =
-        launch_rows_energy(s->d_psi.as<float>(), s->img, x_any_rows_per_wg(r.plan->px), center_of(s, 0, 1),
-                           energy_of(s, 0), st);
+        launch_rows_energy(s->d_psi.as<float>(), s->img, r.geom.eff_local.x, energy_pieces(r.plan->q.x),
+                           x_any_rows_per_wg(r.plan->px), center_of(s, 0, 1), energy_of(s, 0), st);
     if (e != hipSuccess) return e;
   }
   return launch_x_forward_any(*r.plan, r.geom, s->d_psi.as<float>(), kGatherMirror, r.rows.as<float2>(), st,
