@@ -175,7 +175,8 @@ enum {
   MVD_FFT_POW2 = 1,     /* smallest power of two per axis (up to 1024) */
   MVD_FFT_AUTOTUNE = 2  /* time the smallest 5-smooth size and the smallest size of the register-resident
                            kernels (64, 128, 144, 192, 256, 288, 384, 512; twice those along x) per axis
-                           on the GPU, keep the fastest shape (cached per window shape) */
+                           on the GPU, keep the fastest shape (cached per window shape); done for
+                           iterations in block windows, else as MVD_FFT_SMOOTH */
 };
 
 /* new MVDeconInput + image geometry: nviews views of nx*ny*nz voxels on `device`. */

@@ -1994,9 +1994,9 @@ int tune_fft_shape(mvd_session* s, Int3 win, Int3* q, float* ms_out) {
   return 0;
 }
 
-int choose_fft_shape(mvd_session* s, Int3 win, Int3* q) {
+int choose_fft_shape(mvd_session* s, Int3 win, bool tune, Int3* q) {
   const Int3 smooth = fft_shape_for(win);
-  if (s->fft_policy == MVD_FFT_SMOOTH) {
+  if (s->fft_policy == MVD_FFT_SMOOTH || (s->fft_policy == MVD_FFT_AUTOTUNE && !tune)) {
     *q = smooth;
     return 0;
   }
@@ -2054,13 +2054,16 @@ int choose_blocks(mvd_session* s, Int3 kd, Int3* bs_out, Int3* q_out) {
   return 0;
 }
 
-int build_geometry(mvd_session* s, int v) {
+// tune: MVD_FFT_AUTOTUNE times shapes and splits (of the iteration in block
+// windows: sessions by rows leave them alone); else it takes the smallest
+// 5-smooth sizes.
+int build_geometry(mvd_session* s, int v, bool tune) {
   mvd_session::View& view = s->views[v];
   Int3 bs = s->use_blocks ? s->block
                           : Int3{s->img.x + view.kd.x - 1, s->img.y + view.kd.y - 1, s->img.z + view.kd.z - 1};
   Int3 q;
-  int rc0 = !s->use_blocks && s->fft_policy == MVD_FFT_AUTOTUNE ? choose_blocks(s, view.kd, &bs, &q)
-                                                                : choose_fft_shape(s, bs, &q);
+  int rc0 = !s->use_blocks && s->fft_policy == MVD_FFT_AUTOTUNE && tune ? choose_blocks(s, view.kd, &bs, &q)
+                                                                        : choose_fft_shape(s, bs, tune, &q);
   if (rc0) return rc0;
   view.plan = s->plans.get(q);
   if (!view.plan) return -1;
@@ -2113,8 +2116,8 @@ int use_windows(mvd_session* s) {
   s->bb.built = false;
   ++s->epoch;
   for (int v = 0; v < s->nviews; ++v) {
-    int rc = view_spectra(s, v);
-    if (rc) return rc;
+    int rc = s->fft_policy == MVD_FFT_AUTOTUNE ? build_geometry(s, v, true) : 0;
+    if (rc || (rc = view_spectra(s, v))) return rc;
   }
   int rc = ensure_workspace(s);
   if (rc) return rc;
@@ -2402,10 +2405,14 @@ int mvd_prepare(mvd_session* s, int psf_type, double lambda, const int* block_xy
   // MVDeconInput.init: views in order
   if (int rc = init_views(s, false)) return rc;
   for (int v = 0; v < s->nviews; ++v) {
-    int rc = build_geometry(s, v);
+    int rc = build_geometry(s, v, false);
     if (rc) return rc;
   }
   if (int rc = plan_rows(s)) return rc;
+  for (int v = 0; s->fft_policy == MVD_FFT_AUTOTUNE && !s->rc.on && v < s->nviews; ++v) {
+    int rc = build_geometry(s, v, true);
+    if (rc) return rc;
+  }
   for (int v = 0; v < s->nviews; ++v) {
     int rc = view_spectra(s, v);
     if (rc) return rc;
