@@ -728,6 +728,11 @@ struct mvd_session {
     DeviceBuf kern, spec, work, a, b, out;
     LaunchTables tables;
     std::vector<PassLaunch> kernels, conv;
+    size_t bytes() const {
+      size_t n = 0;
+      for (const DeviceBuf* x : {&kern, &spec, &work, &a, &b, &out}) n += x->bytes;
+      return n;
+    }
   } cp;
   PlanCache plans;
   Timer timer;
@@ -1709,6 +1714,11 @@ int init_view(mvd_session* s, int v, bool normalise = true) {
   return 0;
 }
 
+// Most workspace of the compound kernels (up to 512 MiB of spectra) that a
+// session holds which has prepared them once: four views with 25x25x31 kernels
+// take 25 MB; six with 41x41x81 kernels would hold 396 MiB in all, not 82.
+constexpr size_t kKeptCompound = size_t(64) << 20;
+
 // MVDeconFFT.init of all views at once, k1 holding the kernels as given: view v
 // is prepared from its own normalised kernel1, the normalised ones of the views
 // before it, and of the views after it the ones as given (normalise_first
@@ -2404,6 +2414,8 @@ int mvd_prepare(mvd_session* s, int psf_type, double lambda, const int* block_xy
   for (auto& v : s->views) v.k1 = v.psf_raw;
   // MVDeconInput.init: views in order
   if (int rc = init_views(s, false)) return rc;
+  // (a session that sets its PSFs again keeps the workspace from then on)
+  if (s->cp.bytes() > kKeptCompound) s->cp = mvd_session::Compound();
   for (int v = 0; v < s->nviews; ++v) {
     int rc = build_geometry(s, v, false);
     if (rc) return rc;
