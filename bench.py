@@ -805,8 +805,7 @@ def main():
     q = geo["fft"]
     effs = block_effective_sizes(w["size_xyz"], w["k_xyz"], blk) if blk else [tuple(w["size_xyz"])]
     kb = kernel_bytes(effs, q, n)
-    # by rows the forward x pass runs once per call, not once per convolution
-    by_rows = max(tim.get(c, (0, 0))[1] for c in ("x_forward", "xy_forward")) < nv * timed_iters
+    by_rows = d.by_rows
     if by_rows:
         kb = row_kernel_bytes(w["size_xyz"], w["k_xyz"])
         win = [a + b - 1 for a, b in zip(w["size_xyz"], w["k_xyz"])]
@@ -887,7 +886,8 @@ def main():
                                f"{w['size_xyz'][2]} f32, PSF {w['k_xyz'][0]}x{w['k_xyz'][1]}x{w['k_xyz'][2]}, "
                                f"blocks {blk}, lambda {w['lam']}, efficient-Bayesian, precomputed weights",
                    "views": nv, "size_xyz": list(w["size_xyz"]), "block": list(blk) if blk else None,
-                   "fft_shape": list(q), "parallelism": "single GPU"},
+                   "iteration": "by rows" if by_rows else "block windows",
+                   "fft_shape": None if by_rows else list(q), "parallelism": "single GPU"},
         "roofline": {"bound": "hbm", "kernel": dom, "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS,
                      "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": traffic,
                      "avg_launch_us": round(dc["avg_us"], 2)},
