@@ -1,5 +1,5 @@
 // Two-pass register FFT for any 5-smooth length that splits into two radices
-// of at most 32 (every such length up to 960, and 1024), with the radices
+// of at most 32 (all up to 1024 but 2, 3, 5, 972 and 1000), with the radices
 // chosen at run time.
 //
 // A length N = A B is transformed in two passes.  In the first, B threads per
@@ -13,7 +13,7 @@
 //
 // This replaced a pass per radix 2, 3, 4, 5 or 8 over lines held in LDS (four
 // to five LDS sweeps and barriers a transform), which remains for the lengths
-// without such a split (972 and 1000, and below 4).  Measured per launch,
+// without such a split.  Measured per launch,
 // before and after: x inverse with the quotient, rows of 360 samples, 263 x 149
 // rows: 126 -> 54 us; x forward there 108 -> 33 us; y of 150 points, 76 columns
 // x 96 planes: 15 -> 8 us.  Ten iterations of three 128x128x64 views (150 x 150

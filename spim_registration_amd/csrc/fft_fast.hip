@@ -1232,11 +1232,6 @@ hipError_t launch_y_fast_window(const ShapePlan& sp, float2* spec, int zlo, int 
   return hipGetLastError();
 }
 
-hipError_t launch_y_fast(const ShapePlan& sp, float2* spec, int zlo, int zhi, int ylo, int yhi, float dir,
-                         hipStream_t stream) {
-  return launch_y_fast_window(sp, spec, zlo, zhi, ylo, yhi, dir, {0, 0, 0}, {1 << 30, 1 << 30, 1 << 30}, stream);
-}
-
 hipError_t launch_z_fast(const ShapePlan& sp, float2* spec, const float2* kspec, float scale, int zlo, int zhi,
                          hipStream_t stream, float dir, float2* aux, const float2* pre, const double* wsum,
                          double kdc) {

@@ -474,7 +474,7 @@ __global__ __launch_bounds__(kEnergyThreads) void k_energy_check(const EnergyIte
         sq += sums[3 * i];
         n += sums[3 * i + 1];
       }
-      if (!(mean * n <= E.limit * sq)) refuse = 1;
+      if (!(mean * n < E.limit * sq)) refuse = 1;
     }
   }
   refuse = __syncthreads_or(refuse);

@@ -287,7 +287,7 @@ __global__ __launch_bounds__(kGThreads) void k_window_sum(const float* img, Int3
   constexpr int kFly = 8;
   __shared__ double rs[kGThreads];
   __shared__ int cnt[kGThreads + kFly];
-  const int nrows = n.y * n.z;  // (launch_window_sum_to)
+  const int nrows = n.y * n.z;  // (an image has fewer than 2^31 voxels)
   const int per = (nrows + gridDim.x - 1) / gridDim.x;
   const int64_t first = (int64_t)blockIdx.x * per;
   const int r0 = (int)(first < nrows ? first : nrows), r1 = nrows - r0 < per ? nrows : r0 + per;

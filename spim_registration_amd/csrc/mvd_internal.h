@@ -339,8 +339,6 @@ hipError_t launch_x_inverse_any(const ShapePlan& sp, const ConvGeom& g, const fl
 bool fast_size(int n);
 inline bool register_size(const FftPlan& p) { return fast_size(p.n) || any_size(p); }
 int x_fast_rows_per_wg(int M);
-hipError_t launch_y_fast(const ShapePlan& sp, float2* spec, int zlo, int zhi, int ylo, int yhi, float dir,
-                         hipStream_t stream);
 hipError_t launch_y_fast_window(const ShapePlan& sp, float2* spec, int zlo, int zhi, int ylo, int yhi, float dir,
                                 Int3 in_lo, Int3 in_hi, hipStream_t stream);
 hipError_t launch_z_fast(const ShapePlan& sp, float2* spec, const float2* kspec, float scale, int zlo, int zhi,
