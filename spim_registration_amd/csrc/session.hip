@@ -757,13 +757,13 @@ struct mvd_session {
   // transforms the new row forward again, ready for the next convolution.
   // Against block windows this stores no row or plane twice, pads the image
   // once instead of every block, and takes one pass less per convolution; the
-  // ratio image never reaches memory.  Blocked and whole convolutions are one
-  // operator, so only rounding depends on it.  Ten iterations of 6 views of
-  // 512x512x256 in 256^3 blocks (18 windows, 4.5 times the image's voxels)
-  // 156 -> 112 ms, five of 3 views of 421x337x203 in 192^3 blocks 24.6 -> 15.2
-  // ms, of four 311x263x149 views in one window 18.7 -> 16.2 ms.  The y passes
-  // run at 5.5 to 5.9 TB/s; the z pass (3.5 TB/s) and the x pass (3.6) are held
-  // by VALU issue (55 %) and the latency of their three exchanges together.
+  // ratio image never reaches memory.  Ten iterations of 6 views of 512x512x256
+  // in 256^3 blocks (18 windows, 4.5 times the image's voxels) 156 -> 115 ms,
+  // five of 3 views of 421x337x203 in 192^3 blocks 24.6 -> 15.2 ms, ten of four
+  // 311x263x149 views in one window 18.7 -> 16.1 ms.  The y passes move 5.5 to
+  // 5.7 TB/s; in the x passes (3.4 TB/s) a SIMD issues VALU instructions 56 to
+  // 63 % of the time, with 3.6 waves, in the z pass (3.3 TB/s) 50 % with 1.9;
+  // the rest is the latency of their exchanges.
   //
   // One value that is no finite number reaches every value of its rows, then of
   // its tile: in block windows it reaches its blocks, in one window the image.
