@@ -1144,6 +1144,31 @@ void drop_rows(mvd_session* s) {
   }
 }
 
+// All buffers of the iteration by rows that plan_rows has chosen, so that what
+// later sessions see as free is free; false where one cannot be had.
+bool reserve_rows(mvd_session* s) {
+  auto& r = s->rc;
+  const Int3 n = s->img;
+  const size_t nrows = (size_t)n.y * n.z, convs = r.guard ? 2 * (size_t)s->nviews : 0;
+  const size_t spec = r.shared ? 0 : sizeof(float2) * slab_elems(*r.plan, r.plan->q.z);
+  std::vector<std::pair<DeviceBuf*, size_t>> sizes = {
+      {&r.rows, sizeof(float2) * r.plan->pitch * (nrows + 1)},
+      {&r.planes, sizeof(float2) * (slab_elems(*r.plan, n.z) * r.tiles.size() + slab_elems(*r.plan, 1))},
+      {&r.energy, sizeof(float2) * convs * r.nwg * energy_pieces(r.plan->q.x)},
+      {&r.esums, r.guard ? sizeof(double) * (3 * convs * r.regions * r.slices + 1) : 0},
+      {&r.plain, r.shared ? 0 : sizeof(float2) * r.plan->spectrum_elems()}};
+  for (auto& v : s->views) {
+    sizes.push_back({&v.r1hat, spec});
+    sizes.push_back({&v.r2hat, spec});
+  }
+  for (auto& b : sizes)
+    if (b.first->ensure(b.second) != hipSuccess) {
+      (void)hipGetLastError();
+      return false;
+    }
+  return true;
+}
+
 // Chooses the whole-image iteration of a prepared session (RowConv): needs one
 // kernel size for all views (they share the rows), lengths with two-radix
 // kernels, and its buffers in half of the free memory; otherwise the blocks are
@@ -1243,15 +1268,7 @@ int plan_rows(mvd_session* s) {
   r.guard = split || r.tiles.size() > 1;
   r.centred = split;
   r.on = true;
-  if (r.shared) return 0;
-  // the kernels' spectra now, the rest at the first iteration (reserve_rows)
-  bool have_mem = r.plain.ensure(sizeof(float2) * r.plan->spectrum_elems()) == hipSuccess;
-  for (auto& v : s->views)
-    have_mem = have_mem && v.r1hat.ensure(spec_b) == hipSuccess && v.r2hat.ensure(spec_b) == hipSuccess;
-  if (!have_mem) {
-    (void)hipGetLastError();
-    drop_rows(s);
-  }
+  if (!reserve_rows(s)) drop_rows(s);
   return 0;
 }
 
@@ -1378,29 +1395,8 @@ void rows_pass_descs(mvd_session* s, int v, int conv, std::vector<RowsPass> (&pa
   xinv->push_back(x);
 }
 
-// Buffers of the iteration by rows.  They are allocated at the first iteration
-// (a session may never iterate), when the memory that plan_rows saw may be
-// gone: false, and the caller goes on in block windows.
-bool reserve_rows(mvd_session* s) {
-  auto& r = s->rc;
-  if (r.consts) return true;
-  const Int3 n = s->img;
-  const size_t nrows = (size_t)n.y * n.z, convs = r.guard ? 2 * (size_t)s->nviews : 0;
-  const std::pair<DeviceBuf*, size_t> sizes[] = {
-      {&r.rows, sizeof(float2) * r.plan->pitch * (nrows + 1)},
-      {&r.planes, sizeof(float2) * (slab_elems(*r.plan, n.z) * r.tiles.size() + slab_elems(*r.plan, 1))},
-      {&r.energy, sizeof(float2) * convs * r.nwg * energy_pieces(r.plan->q.x)},
-      {&r.esums, r.guard ? sizeof(double) * (3 * convs * r.regions * r.slices + 1) : 0}};
-  for (auto& b : sizes)
-    if (b.first->ensure(b.second) != hipSuccess) {
-      (void)hipGetLastError();
-      return false;
-    }
-  return true;
-}
-
 // The spectra of the constant one that the ratio has outside the image (zero
-// where it is centred): a row along x, a plane along x and y.  After reserve_rows.
+// where it is centred): a row along x, a plane along x and y.
 int ensure_rows(mvd_session* s) {
   auto& r = s->rc;
   if (r.consts) return 0;
@@ -1452,15 +1448,11 @@ hipError_t restore_psi(mvd_session* s, hipStream_t st) {
   return hipMemcpyAsync(s->d_psi.p, s->d_ratio.p, sizeof(float) * s->n, hipMemcpyDeviceToDevice, st);
 }
 
-int use_windows(mvd_session* s);
-
 // Launch lists of the block-batched iteration (one spectrum buffer per block).
 // Off for single-block views and when the extra spectra would take more than
 // half of the free device memory.
 int build_block_batch(mvd_session* s) {
   auto& bb = s->bb;
-  if (s->rc.on && !reserve_rows(s))
-    if (int rc = use_windows(s)) return rc;
   bb.view.clear();
   bb.ztab.clear();
   bb.tables.host.clear();
@@ -1494,8 +1486,11 @@ int build_block_batch(mvd_session* s) {
   const size_t need = nb * elems * sizeof(float2);
   bb.built = true;
   bb.enabled = nb > 1 && need <= bb.arena.bytes + free_b / 2;
+  if (bb.enabled && bb.arena.ensure(need) != hipSuccess) {
+    (void)hipGetLastError();
+    bb.enabled = false;
+  }
   if (!bb.enabled) return 0;
-  MVD_CHECK(bb.arena.ensure(need));
   MVD_CHECK(hipMemsetAsync(bb.arena.p, 0, need, s->stream));  // finite row padding
   std::vector<float2*> spec;
   for (size_t b = 0; b < nb; ++b) spec.push_back(bb.arena.as<float2>() + b * elems);
@@ -2121,7 +2116,9 @@ int ensure_workspace(mvd_session* s) {
 
 // Leaves the iteration by rows for good: its buffers go, the block windows'
 // spectra and workspace are made.  Nothing may run on the session's buffers.
+// Where that fails the session has to be prepared again.
 int use_windows(mvd_session* s) {
+  s->prepared = false;
   drop_rows(s);
   s->bb.built = false;
   ++s->epoch;
@@ -2132,6 +2129,7 @@ int use_windows(mvd_session* s) {
   int rc = ensure_workspace(s);
   if (rc) return rc;
   MVD_CHECK(hipStreamSynchronize(s->stream));
+  s->prepared = true;
   return 0;
 }
 
@@ -2421,6 +2419,7 @@ int mvd_prepare(mvd_session* s, int psf_type, double lambda, const int* block_xy
     if (rc) return rc;
   }
   if (int rc = plan_rows(s)) return rc;
+  if (!s->rc.on) drop_rows(s);
   for (int v = 0; s->fft_policy == MVD_FFT_AUTOTUNE && !s->rc.on && v < s->nviews; ++v) {
     int rc = build_geometry(s, v, true);
     if (rc) return rc;
@@ -3072,8 +3071,6 @@ int build_batch(mvd_batch* b) {
   int maxv = 0, tot = 0;
   for (auto* s : b->stacks) {
     MVD_REQUIRE(s->prepared, "a session is not prepared");
-    if (s->rc.on && !reserve_rows(s))
-      if (int rc = use_windows(s)) return rc;
     b->stats_off.push_back(tot);
     tot += 2 * s->nviews;
     maxv = std::max(maxv, s->nviews);
